@@ -5,9 +5,11 @@ Each case is one call, or one training step, of the Python entry points
 the GPU.  ``B`` is batch times heads (the heads are folded into the batch),
 ``mode`` what the program does with the op:
 
-  fwd    the forward alone, as inference does;
-  bwd    the gradient alone, given the forward's results;
-  train  ``sdpa_autograd`` and the gradients of q, k and v.
+  fwd       the forward alone, as inference does;
+  bwd       the gradient alone, given the forward's results;
+  train     the forward op and then the gradient op, as a training program
+            that holds both ops calls them;
+  autograd  the same step through ``sdpa_autograd`` and torch's backward.
 
 ``draw`` gives further cases of the same kinds over the sizes that each kind
 has in use.
@@ -40,7 +42,7 @@ def listed():
         # Reading a prompt of odd length: 2 sequences with 16 heads.
         ("prefill_f16", _case("prefill", "fwd", "f16", 32, 1999, 1999, 128, 128, True, 0.0)),
         # A layer of a long-sequence model with 64-wide heads, trained without dropout.
-        ("train_f16_d64", _case("self", "train", "f16", 256, 2048, 2048, 64, 64, True, 0.0)),
+        ("train_f16_d64", _case("self", "autograd", "f16", 256, 2048, 2048, 64, 64, True, 0.0)),
         # The benchmark's workload, forward and gradient apart: the largest
         # half-precision calls.
         ("forward_f16_d128", _case("self", "fwd", "f16", 128, 4096, 4096, 128, 128, True, 0.1)),
@@ -103,7 +105,7 @@ def draw(rng):
         B, S_q = _log(rng, 8, 128), _log(rng, 100, 8192)
         S_kv = S_q
     elif kind == "self":
-        mode = rng.choice(["train", "train", "fwd", "bwd"])
+        mode = rng.choice(["train", "autograd", "fwd", "bwd"])
         causal = rng.random() < 0.7
         B, S_q = _log(rng, 8, 256), _log(rng, 128, 4096)
         S_kv = S_q
@@ -143,7 +145,7 @@ def prepare(case, seed):
     state = {"op": op, "mode": c["mode"], "q": q, "k": k, "v": v, "d_o": d_o, "args": args, "attrs": attrs}
     if c["mode"] == "bwd":
         state["o"], state["stats"] = op.sdpa(q, k, v, *args, **attrs)
-    elif c["mode"] == "train":
+    elif c["mode"] == "autograd":
         for t in (q, k, v):
             t.requires_grad_(True)
     return state
@@ -155,6 +157,9 @@ def run(state):
         return op.sdpa(q, k, v, *state["args"], **state["attrs"])
     if state["mode"] == "bwd":
         return op.sdpa_grad(q, k, v, state["o"], state["stats"], state["d_o"], *state["args"], **state["attrs"])
+    if state["mode"] == "train":
+        o, stats = op.sdpa(q, k, v, *state["args"], **state["attrs"])
+        return (o, stats) + op.sdpa_grad(q, k, v, o, stats, state["d_o"], *state["args"], **state["attrs"])
     o, stats = op.sdpa_autograd(q, k, v, *state["args"], **state["attrs"])
     return (o.detach(), stats) + torch.autograd.grad(o, (q, k, v), state["d_o"])
 
