@@ -106,6 +106,20 @@ int sdpa_hip_fwd(int dtype, const void* q, const void* k, const void* v, void* o
                  int B, int S_q, int S_kv, int D_qk, int D_v, float scale, float dropout,
                  int causal_mask, uint64_t seed, uint64_t offset, hipStream_t stream);
 
+/* The same with a workspace.  Where the query side has too few tiles to fill
+ * the GPU (token generation, a few queries against a long memory) the keys
+ * of a tile are divided over several workgroups, which needs
+ * sdpa_hip_fwd_workspace_bytes(...) bytes of device memory, 16-byte aligned,
+ * for their partial results; 0 where nothing is divided.  With less (or
+ * none) the call runs undivided, as sdpa_hip_fwd does.                      */
+size_t sdpa_hip_fwd_workspace_bytes(int dtype, int B, int S_q, int S_kv, int D_qk, int D_v,
+                                    int causal_mask);
+
+int sdpa_hip_fwd_ws(int dtype, const void* q, const void* k, const void* v, void* o, float* stats,
+                    void* workspace, size_t workspace_bytes, int B, int S_q, int S_kv, int D_qk,
+                    int D_v, float scale, float dropout, int causal_mask, uint64_t seed,
+                    uint64_t offset, hipStream_t stream);
+
 /* ---- backward: replaces FlashAttnGradFunctor<GPUDevice,T> (sdpa/sdpa_bwd.cu.cc:347-453)
  * Needs a device workspace of sdpa_hip_bwd_workspace_bytes(B, S_q) bytes
  * (two fp32 values per query row: stats * log2(e) and delta = sum_d dO * O),

@@ -1,0 +1,54 @@
+"""Shapes with too few tiles to fill the GPU: the forward kernel of 32-query
+tiles (csrc/sdpa_f16_fwd_small.hip), its division of a tile's keys over
+workgroups, and the edges of both against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from _common import TOL, Cfg, make_inputs, maxabs, oracle_kw
+from test_parity_gpu import _np, _t, run_and_check
+
+pytestmark = pytest.mark.gpu
+
+FWD = [
+    # B, S_q, S_kv, D_qk, D_v, causal, dropout; parts of a tile's keys
+    (2, 1, 1, 64, 64, False, 0.0, 1),        # one block, one wave
+    (3, 33, 97, 40, 72, False, 0.1, 1),      # a block more than the waves, ragged widths
+    (2, 129, 129, 128, 128, True, 0.1, 1),   # the diagonal block, a one-row tile
+    (1, 31, 1551, 128, 64, False, 0.2, 6),   # parts of unequal length, a ragged tail
+    (2, 32, 4096, 32, 128, False, 0.0, 16),  # two blocks per wave
+    (5, 2, 3001, 64, 64, False, 1.5, 12),    # every element dropped
+]
+
+
+@pytest.mark.parametrize("case", FWD, ids=["-".join(map(str, c)) for c in FWD])
+def test_small_forward(pkg, O, case):
+    B, S_q, S_kv, D_qk, D_v, causal, p, parts = case
+    c = Cfg("small_fwd", "f16", B, S_q, S_kv, D_qk, D_v, causal, p, D_qk ** -0.5, 3, 17)
+    L = pkg.library()
+    rows = parts * B * S_q
+    want = 0 if parts == 1 else (rows * D_v * 4 + 255) // 256 * 256 + rows * 8
+    dims = (1, B, S_q, S_kv, D_qk, D_v, int(causal))
+    assert L.sdpa_hip_fwd_workspace_bytes(*dims) == want
+    run_and_check(pkg, O, c)
+
+    # a workspace one byte short, or none, runs undivided: the same bits
+    q, k, v = (_t(a) for a in make_inputs(c)[:3])
+    outs = []
+    for ws_bytes in (want, max(want - 1, 0), 0):
+        ws = torch.empty((max(want, 1),), dtype=torch.uint8, device=q.device)
+        o = torch.empty((B, S_q, D_v), dtype=q.dtype, device=q.device)
+        s = torch.empty((B, S_q), dtype=torch.float32, device=q.device)
+        rc = L.sdpa_hip_fwd_ws(1, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), s.data_ptr(),
+                               ws.data_ptr(), ws_bytes, B, S_q, S_kv, D_qk, D_v, c.scale, p, int(causal), c.seed,
+                               c.offset, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        outs.append((_np(o), _np(s)))
+    for a, b in zip(outs[1], outs[2]):
+        assert np.array_equal(a, b)
+    # Both forms against the oracle at the op's tolerance (they round P~ to
+    # half relative to different running maxima, so their bits differ).
+    o_ref, s_ref = O.sdpa_fwd_gate(*make_inputs(c)[:3], **oracle_kw(c))
+    for o, s in (outs[0], outs[2]):
+        assert maxabs(o, o_ref) <= TOL["f16"]["o"] and maxabs(s, s_ref) <= TOL["f16"]["stats"]

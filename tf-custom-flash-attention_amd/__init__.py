@@ -73,6 +73,11 @@ def library():
     L.sdpa_hip_fwd.restype = i32
     L.sdpa_hip_fwd.argtypes = [i32, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, f32, f32, i32,
                                u64, u64, vp]
+    L.sdpa_hip_fwd_workspace_bytes.restype = sz
+    L.sdpa_hip_fwd_workspace_bytes.argtypes = [i32] * 7
+    L.sdpa_hip_fwd_ws.restype = i32
+    L.sdpa_hip_fwd_ws.argtypes = [i32, vp, vp, vp, vp, vp, vp, sz, i32, i32, i32, i32, i32, f32, f32, i32,
+                                  u64, u64, vp]
     L.sdpa_hip_bwd_workspace_bytes.restype = sz
     L.sdpa_hip_bwd_workspace_bytes.argtypes = [i32, i32]
     L.sdpa_hip_bwd.restype = i32
@@ -188,10 +193,13 @@ def sdpa(q, k, v, seed=0, offset=0, dropout: float = 0.0, scale: float = 1.0,
     S_kv, D_v = k.shape[1], v.shape[2]
     o = torch.empty((B, S_q, D_v), dtype=q.dtype, device=q.device)
     stats = torch.empty((B, S_q), dtype=torch.float32, device=q.device)
-    rc = library().sdpa_hip_fwd(dt, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                stats.data_ptr(), B, S_q, S_kv, D_qk, D_v, float(scale),
-                                float(dropout), int(bool(causal_mask)), _u64(seed), _u64(offset),
-                                _stream_handle(q.device))
+    L = library()
+    ws_bytes = L.sdpa_hip_fwd_workspace_bytes(dt, B, S_q, S_kv, D_qk, D_v, int(bool(causal_mask)))
+    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=q.device) if ws_bytes else None
+    rc = L.sdpa_hip_fwd_ws(dt, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), stats.data_ptr(),
+                           ws.data_ptr() if ws_bytes else None, ws_bytes, B, S_q, S_kv, D_qk, D_v,
+                           float(scale), float(dropout), int(bool(causal_mask)), _u64(seed), _u64(offset),
+                           _stream_handle(q.device))
     _raise_for(rc)
     return o, stats
 

@@ -11,6 +11,7 @@
 #include "sdpa_device.h"
 #include "sdpa_launch.h"
 #include "sdpa_params.h"
+#include "sdpa_parts.h"
 
 namespace {
 
@@ -122,9 +123,22 @@ int sdpa_hip_check_bwd(int q_rank, const int64_t* q, int k_rank, const int64_t* 
                                   seed_rank, offset_rank, causal_mask);
 }
 
+size_t sdpa_hip_fwd_workspace_bytes(int dtype, int B, int S_q, int S_kv, int D_qk, int D_v, int causal_mask) {
+    if (check_common(dtype, B, S_q, S_kv, D_qk, D_v, 0.f, causal_mask) != SDPA_OK) return 0;
+    return sdpa::fwd_plan(dtype == SDPA_DTYPE_F16, B, S_q, S_kv, D_qk, D_v, causal_mask != 0).bytes;
+}
+
 int sdpa_hip_fwd(int dtype, const void* q, const void* k, const void* v, void* o, float* stats,
                  int B, int S_q, int S_kv, int D_qk, int D_v, float scale, float dropout,
                  int causal_mask, uint64_t seed, uint64_t offset, hipStream_t stream) {
+    return sdpa_hip_fwd_ws(dtype, q, k, v, o, stats, nullptr, 0, B, S_q, S_kv, D_qk, D_v, scale, dropout,
+                           causal_mask, seed, offset, stream);
+}
+
+int sdpa_hip_fwd_ws(int dtype, const void* q, const void* k, const void* v, void* o, float* stats,
+                    void* workspace, size_t workspace_bytes, int B, int S_q, int S_kv, int D_qk, int D_v,
+                    float scale, float dropout, int causal_mask, uint64_t seed, uint64_t offset,
+                    hipStream_t stream) {
     int st = check_common(dtype, B, S_q, S_kv, D_qk, D_v, dropout, causal_mask);
     if (st != SDPA_OK) return st;
     if ((size_t)B * S_q == 0) return SDPA_OK;  // empty grid: nothing to do
@@ -139,7 +153,15 @@ int sdpa_hip_fwd(int dtype, const void* q, const void* k, const void* v, void* o
     p.s = sdpa::AttnShape{B, S_q, S_kv, D_qk, D_v};
     p.c = make_scalars(scale, dropout, causal_mask, seed, offset, false);
     const bool vec = vec_ok(dtype, D_qk, D_v, {q, k, v, o});
-    if (dtype == SDPA_DTYPE_F16 && vec) return hip_status(sdpa::launch_fwd_f16_dma(p, stream));
+    const sdpa::FwdPlan plan = sdpa::fwd_plan(dtype == SDPA_DTYPE_F16, B, S_q, S_kv, D_qk, D_v, causal_mask != 0);
+    p.parts = 1;
+    if (plan.bytes > 0 && workspace && aligned16(workspace) && workspace_bytes >= plan.bytes) {
+        p.parts = plan.parts;
+        p.part_o = static_cast<float*>(workspace);
+        p.part_ml = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + plan.o_bytes);
+    }
+    if (dtype == SDPA_DTYPE_F16 && vec)
+        return hip_status(plan.small ? sdpa::launch_fwd_f16_wave(p, stream) : sdpa::launch_fwd_f16_dma(p, stream));
     return hip_status(sdpa::launch_fwd(p, (sdpa::DType)dtype, vec, stream));
 }
 

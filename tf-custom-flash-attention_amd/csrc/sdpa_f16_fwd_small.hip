@@ -1,0 +1,363 @@
+// sdpa_f16_fwd_small.hip -- fp16 Sdpa forward for gfx950 where the query side
+// has too few tiles to fill the chip: token generation, a few queries against
+// a long memory, short sequences, few heads.
+//
+// The kernel of sdpa_f16_fwd.hip gives a workgroup 128 queries and all of
+// their keys; with few such tiles most of the 256 CUs idle, and each busy one
+// runs a long serial chain of key blocks.  Here a workgroup owns 32 queries,
+// its four waves take the 32-key blocks in turn, each wave with running
+// statistics and an accumulator of its own (merged through LDS at the end),
+// and the blocks of one tile may further be divided over several workgroups
+// (sdpa_parts.h), whose results a second kernel merges from the caller's workspace.
+//
+// Each wave streams its own K/V blocks through a two-stage LDS ring (the
+// copies of sdpa_dma.h): no two waves share a block, so the loop has no
+// barrier, only waits on the wave's own copies.  The price is that the K/V
+// rows go to LDS once per 32 queries instead of once per 128.
+//
+// Element semantics are those of sdpa_f16_fwd.hip (hi/lo split of P~
+// included; its test sees the mass of this wave's earlier keys only, which
+// errs towards splitting).
+#include "sdpa_dma.h"
+#include "sdpa_launch.h"
+#include "sdpa_params.h"
+#include "sdpa_parts.h"
+
+namespace sdpa {
+namespace {
+
+constexpr float kTauW = 8.0f;  // lazy-rescale threshold (log2 units), as in sdpa_f16_fwd.hip
+
+// Copies of one 32 x (8 L) fp16 tile by a single wave: copy u fills LDS chunk
+// slots 64 u + lane, i.e. rows 64 u / L + lane / L.  The swizzle repeats every
+// PERIOD copies (TR: the swz_tr layout of tiles read only transposed).
+template <int L, bool TR>
+struct WaveCopy {
+    static constexpr int LOADS = L / 2, RPC = 64 / L;
+    static constexpr int PERIOD = TR || RPC >= 16 ? 1 : 16 / RPC;
+    static constexpr int NV = PERIOD < LOADS ? PERIOD : LOADS;
+    uint32_t voff[NV];
+    __device__ __forceinline__ void init(int lane, int row_bytes, int valid_chunks) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            const int r = RPC * u + lane / L;
+            const int c = (lane % L) ^ (TR ? swz_tr<L>(r) : swz<L>(r));
+            voff[u] = c < valid_chunks ? (uint32_t)(r * row_bytes + c * 16) : kOob;
+        }
+    }
+    __device__ __forceinline__ void issue(const RowSrc& src, uint32_t m0) const {
+        const rsrc_t rs = src.at(0);
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u)
+            dma16_at(rs, m0 + 1024u * u, voff[u % NV] + (uint32_t)((u / NV) * NV * RPC * src.row_bytes));
+    }
+};
+
+// s_waitcnt that the compiler does not move LDS reads across: the copies it
+// waits for are invisible to it, and here no barrier follows.
+template <int N>
+__device__ __forceinline__ void wait_copies() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+template <int DQK, int DV>
+struct FwdWaveCfg {
+    static constexpr int NW = 4, NT = 64 * NW, BM = 32, BN = 32;
+    static constexpr int LK = DQK / 8, LV = DV / 8;
+    static constexpr int KB = BN * DQK * 2, VB = BN * DV * 2, STAGE = KB + VB, RING = 2 * STAGE;
+    // merge area (after the loop): O of every wave with rows of DV + 4
+    // floats (16 bytes apart modulo the banks), then m and l
+    static constexpr int OS = DV + 4, MERGE = NW * BM * OS * 4 + NW * BM * 8;
+    static constexpr size_t LDS_BYTES = NW * RING > MERGE ? NW * RING : MERGE;
+    static_assert(LDS_BYTES <= 160 * 1024, "gfx950 LDS");
+    static constexpr int WPE = 2 * LDS_BYTES <= 160 * 1024 ? 2 : 1;
+    static constexpr int COPIES = WaveCopy<LK, false>::LOADS + WaveCopy<LV, true>::LOADS;
+    static_assert(COPIES < 64, "vmcnt is 6 bits");
+};
+
+template <int DQK, int DV, bool CAUSAL, bool DROP>
+__global__ __launch_bounds__((FwdWaveCfg<DQK, DV>::NT))
+__attribute__((amdgpu_waves_per_eu(FwdWaveCfg<DQK, DV>::WPE, FwdWaveCfg<DQK, DV>::WPE)))
+void sdpa_fwd_f16_wave_kernel(const FwdParams p, const int win) {
+    using Cfg = FwdWaveCfg<DQK, DV>;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, LK = Cfg::LK, LV = Cfg::LV, NW = Cfg::NW;
+    constexpr int NKS = DQK / 16, NDT = DV / 32;
+
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int B = p.s.B, S_q = p.s.S_q, S_kv = p.s.S_kv, D_qk = p.s.D_qk, D_v = p.s.D_v;
+    const int np = p.parts, items = (S_q + BM - 1) / BM * np;
+    int b, it;
+    xcd_map(blockIdx.x, B * items, items, CAUSAL, win, b, it);
+    const int qt = it / np, part = it - qt * np;
+    const int q0 = qt * BM, my_q = q0 + l32;
+
+    const half_t* Qb = static_cast<const half_t*>(p.q) + (size_t)b * S_q * D_qk;
+    const RowSrc ksrc = row_src(p.k, (size_t)b * S_kv, S_kv, D_qk * 2);
+    const RowSrc vsrc = row_src(p.v, (size_t)b * S_kv, S_kv, D_v * 2);
+
+    // |scale| with negated queries for scale < 0; 1e-30 for 0 (sdpa_f16_fwd.hip)
+    const float sl2_raw = p.c.scale_log2;
+    const bool neg = sl2_raw < 0.f;
+    const float sl2 = (sl2_raw == 0.f) ? 1e-30f : fabsf(sl2_raw);
+
+    // this wave's blocks: lo + wave, lo + wave + NW, ... below hi
+    const int nblk = (min(S_kv, CAUSAL ? q0 + BM : S_kv) + BN - 1) / BN;
+    const int lo = part_begin(nblk, part, np), hi = part_begin(nblk, part + 1, np);
+    const uint32_t ring = lds_base() + (uint32_t)(wave * Cfg::RING);
+    WaveCopy<LK, false> kc;
+    WaveCopy<LV, true> vc;
+    kc.init(lane, D_qk * 2, D_qk / 8);
+    vc.init(lane, D_v * 2, D_v / 8);
+    auto issue = [&](int blk, uint32_t so) {
+        kc.issue(ksrc.shifted(blk * BN), ring + so);
+        vc.issue(vsrc.shifted(blk * BN), ring + so + (uint32_t)Cfg::KB);
+    };
+    half8 qreg[NKS];
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+        half8 v = __builtin_bit_cast(half8, load_row_chunk<half_t, true>(Qb, my_q, S_q, 16 * ks + 8 * hh, D_qk, D_qk));
+        qreg[ks] = neg ? -v : v;
+    }
+    prologue_loads_landed();
+    if (lo + wave < hi) issue(lo + wave, 0);
+
+    SwzLane<LK> swK;
+    swK.init(lane);
+    const uint32_t rkl = ring + swK.row;                          // K rows (^ 32 ks)
+    const uint32_t tvl = ring + Cfg::KB + tr_lane_off<LV>(lane);  // V^T (^ 64 dt)
+
+    floatx16 oacc[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) oacc[dt] = floatx16{};
+    float m_run = kMaxSentinel, l_run = 0.f;
+    // hash of (my_q, key 4 hh of the wave's current block)
+    uint64_t st = DROP ? lcg_state(p.c.seed_offset, (uint64_t)b * S_q + my_q, (uint64_t)S_kv,
+                                   (uint64_t)((lo + wave) * BN + 4 * hh))
+                       : 0;
+    const uint32_t thr = p.c.drop_threshold;
+
+    uint32_t so = 0;
+    for (int blk = lo + wave; blk < hi; blk += NW, so ^= (uint32_t)Cfg::STAGE) {
+        // the other stage's block has been read; the next block's copies go
+        // out there, and this block's have landed once only those are in flight
+        lds_reads_done();
+        if (blk + NW < hi) {
+            issue(blk + NW, so ^ (uint32_t)Cfg::STAGE);
+            wait_copies<Cfg::COPIES>();
+        } else {
+            wait_copies<0>();
+        }
+        const int kv0 = blk * BN;
+        const float split_thr = m_run + fast_log2(xhalf_sum(l_run)) + kSplitLog2;
+        floatx16 s = floatx16{};
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) s = mfma_f16(ld_b128((rkl ^ (uint32_t)(32 * ks)) + so), qreg[ks], s);
+        half8 av[2][NDT];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+                const uint32_t a = (tvl ^ (uint32_t)(64 * dt)) + so + 16 * LV * 16 * j;
+                av[j][dt] = ld_tr8(a, a + 16 * LV * 8);
+            }
+        if (kv0 + BN > S_kv || (CAUSAL && kv0 + BN - 1 > q0)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = kv0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+                if (key >= S_kv || (CAUSAL && key > my_q)) s[r] = -INFINITY;
+            }
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+        mx = xhalf_max(mx) * sl2;
+        const float m_use = (mx > m_run + kTauW) ? fmaxf(m_run, mx) : m_run;
+        const float alpha = fast_exp2(m_run - m_use);
+        float lq[4];
+        float pf[16];
+        uint64_t sg = st;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) pf[4 * g + e] = fast_exp2(__builtin_fmaf(s[4 * g + e], sl2, -m_use));
+            lq[g] = (pf[4 * g] + pf[4 * g + 1]) + (pf[4 * g + 2] + pf[4 * g + 3]);
+            if constexpr (DROP) {
+                uint64_t se = sg;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    pf[4 * g + e] = lcg_keep(se, thr) ? pf[4 * g + e] : 0.f;
+                    se += kLcgMul;
+                }
+                sg += 8 * kLcgMul;
+            }
+        }
+        if constexpr (DROP) st += (uint64_t)(NW * BN) * kLcgMul;
+        if (wave_any(alpha != 1.f)) {
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+        }
+        l_run = __builtin_fmaf(l_run, alpha, (lq[0] + lq[1]) + (lq[2] + lq[3]));
+        m_run = m_use;
+        half8 pb[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            pb[j] = half8_of(pack_h2(pf[8 * j], pf[8 * j + 1]), pack_h2(pf[8 * j + 2], pf[8 * j + 3]),
+                             pack_h2(pf[8 * j + 4], pf[8 * j + 5]), pack_h2(pf[8 * j + 6], pf[8 * j + 7]));
+        if (wave_any(mx > split_thr)) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                float lo8[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) lo8[i] = pf[8 * j + i] - (float)pb[j][i];
+                const half8 pl = half8_of(pack_h2(lo8[0], lo8[1]), pack_h2(lo8[2], lo8[3]),
+                                          pack_h2(lo8[4], lo8[5]), pack_h2(lo8[6], lo8[7]));
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt) oacc[dt] = mfma_f16(av[j][dt], pl, oacc[dt]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) oacc[dt] = mfma_f16(av[j][dt], pb[j], oacc[dt]);
+    }
+
+    // ---- merge the four waves: every ring has been read
+    const float l_tot = xhalf_sum(l_run);
+    __syncthreads();
+    float* mo = reinterpret_cast<float*>(smem);
+    float* mml = mo + NW * BM * Cfg::OS;
+    if (hh == 0) {
+        mml[(wave * BM + l32) * 2] = m_run;
+        mml[(wave * BM + l32) * 2 + 1] = l_tot;
+    }
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<floatx4*>(mo + (wave * BM + l32) * Cfg::OS + 32 * dt + 8 * g + 4 * hh) =
+                (floatx4){oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+    __syncthreads();
+    // one thread per four columns of a row
+    const bool whole = np == 1;
+#pragma unroll
+    for (int i0 = 0; i0 < BM * (DV / 4); i0 += Cfg::NT) {
+        const int i = i0 + tid, row = i / (DV / 4), c = 4 * (i % (DV / 4)), q = q0 + row;
+        if ((BM * (DV / 4) % Cfg::NT && i >= BM * (DV / 4)) || q >= S_q || c >= D_v) continue;
+        float mw[NW], lw[NW], M = kMaxSentinel;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            mw[w] = mml[(w * BM + row) * 2];
+            lw[w] = mml[(w * BM + row) * 2 + 1];
+            M = fmaxf(M, mw[w]);
+        }
+        float L = 0.f;
+        floatx4 acc = floatx4{};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float f = fast_exp2(mw[w] - M);
+            L = __builtin_fmaf(lw[w], f, L);
+            const floatx4 x = *reinterpret_cast<const floatx4*>(mo + (w * BM + row) * Cfg::OS + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(x[e], f, acc[e]);
+        }
+        const size_t grow = (size_t)b * S_q + q;
+        if (whole) {
+            if (c == 0) p.stats[grow] = ((L > 0.f) ? M * kLn2 : kNegInf) + logf(L + kEps);
+            const float inv = (L > kEps) ? p.c.keep_scale / L : 0.f;
+            half4 hv;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) hv[e] = (half_t)(acc[e] * inv);
+            *reinterpret_cast<half4*>(static_cast<half_t*>(p.o) + grow * D_v + c) = hv;
+        } else {
+            const size_t at = (size_t)part * B * S_q + grow;
+            if (c == 0) {
+                p.part_ml[2 * at] = M;
+                p.part_ml[2 * at + 1] = L;
+            }
+            *reinterpret_cast<floatx4*>(p.part_o + at * D_v + c) = acc;
+        }
+    }
+}
+
+// Merge of a row's parts: o = sum_i O_i 2^(m_i - M) / l, stats from M and l.
+// One thread per four columns.
+template <typename T>
+__global__ __launch_bounds__(256) void sdpa_fwd_merge_kernel(const FwdParams p) {
+    const int D_v = p.s.D_v, np = p.parts, cpr = (D_v + 3) / 4;
+    const size_t rows = (size_t)p.s.B * p.s.S_q;
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const size_t row = i / cpr;
+    const int c = 4 * (int)(i - row * cpr);
+    if (row >= rows) return;
+    // eight parts at a time: their loads all go out before the first is used
+    // (one part after the other, each waited out the memory latency)
+    constexpr int U = 8;
+    float M = kMaxSentinel, L = 0.f;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < np; k0 += U) {
+        float m[U], l[U], o[U][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u < np ? k0 + u : np - 1;
+            const size_t at = k * rows + row;
+            m[u] = p.part_ml[2 * at];
+            l[u] = p.part_ml[2 * at + 1];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[u][e] = c + e < D_v ? p.part_o[at * D_v + c + e] : 0.f;
+        }
+        float Mn = M;
+#pragma unroll
+        for (int u = 0; u < U; ++u) Mn = fmaxf(Mn, m[u]);
+        const float a = fast_exp2(M - Mn);
+        L *= a;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] *= a;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float w = k0 + u < np ? fast_exp2(m[u] - Mn) : 0.f;
+            L = __builtin_fmaf(l[u], w, L);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(o[u][e], w, acc[e]);
+        }
+        M = Mn;
+    }
+    if (c == 0) p.stats[row] = ((L > 0.f) ? M * kLn2 : kNegInf) + logf(L + kEps);
+    const float inv = (L > kEps) ? p.c.keep_scale / L : 0.f;
+    T* o = static_cast<T*>(p.o) + row * D_v + c;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (c + e < D_v) o[e] = (T)(acc[e] * inv);
+}
+
+}  // namespace
+
+hipError_t launch_fwd_f16_wave(const FwdParams& p, hipStream_t stream) {
+    const int B = p.s.B, S_q = p.s.S_q;
+    if (B == 0 || S_q == 0) return hipSuccess;
+    return with_dim(p.s.D_qk, [&](auto dqk) {
+        return with_dim(p.s.D_v, [&](auto dv) {
+            return with_bool(p.c.causal != 0, [&](auto c) {
+                return with_bool(p.c.use_dropout != 0, [&](auto d) {
+                    constexpr int DQK = decltype(dqk)::value, DV = decltype(dv)::value;
+                    using Cfg = FwdWaveCfg<DQK, DV>;
+                    static_assert(Cfg::BM == kSmallRows && Cfg::BN == kSmallRows && Cfg::NW == kSmallWaves, "planned by fwd_plan");
+                    const long long n = (long long)((S_q + Cfg::BM - 1) / Cfg::BM) * p.parts * B;
+                    hipError_t err = launch_kernel<sdpa_fwd_f16_wave_kernel<DQK, DV, decltype(c)::value, decltype(d)::value>>(
+                        (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p,
+                        row_window((size_t)p.s.S_kv * (DQK + DV) * 2));
+                    if (err == hipSuccess && p.parts > 1) {
+                        const long long th = (long long)B * S_q * ((p.s.D_v + 3) / 4);
+                        err = launch_kernel<sdpa_fwd_merge_kernel<half_t>>((unsigned)((th + 255) / 256), 256, 0, stream, p);
+                    }
+                    return err;
+                });
+            });
+        });
+    });
+}
+
+}  // namespace sdpa

@@ -59,6 +59,9 @@ hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, int phases, hip
 // sdpa_f16_dkdv.hip).  They require D_qk and D_v to be multiples of 8 and
 // every tensor 16-byte aligned.
 hipError_t launch_fwd_f16_dma(const FwdParams& p, hipStream_t stream);
+// The same for grids too small to fill the chip (sdpa_f16_fwd_small.hip);
+// p.div and the part buffers as planned by fwd_plan().
+hipError_t launch_fwd_f16_wave(const FwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_f16_dma(const BwdParams& p, int phases, hipStream_t stream);
 // dQ phase of launch_bwd_f16_dma (sdpa_f16_dq.hip)
 hipError_t launch_bwd_dq_f16_dma(const BwdParams& p, hipStream_t stream);

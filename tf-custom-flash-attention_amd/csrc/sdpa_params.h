@@ -31,6 +31,11 @@ struct FwdParams {
     const void* v;
     void* o;
     float* stats;
+    // Small grids (sdpa_parts.h): workgroups that share a tile's keys, and
+    // the workspace of their results where there are several
+    int parts;
+    float* part_o;   // [part][B S_q][D_v]: unnormalised O of each part
+    float* part_ml;  // [part][B S_q][2]: its running maximum (log2) and sum
     AttnShape s;
     AttnScalars c;
 };

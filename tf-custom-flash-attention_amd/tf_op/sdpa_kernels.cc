@@ -83,6 +83,15 @@ struct Backend<GPUDevice> {
     static Status fwd(OpKernelContext* ctx, int dt, const void* q, const void* k, const void* v, void* o,
                       float* stats, int B, int S_q, int S_kv, int D_qk, int D_v, float scale, float dropout,
                       bool causal, uint64 seed, uint64 offset) {
+        // Workspace from TF's allocator where the keys of a tile are divided
+        // over workgroups (few query tiles); undivided when it cannot be had.
+        const size_t ws_bytes = sdpa_hip_fwd_workspace_bytes(dt, B, S_q, S_kv, D_qk, D_v, causal ? 1 : 0);
+        if (ws_bytes > 0) {
+            Tensor ws;
+            if (ctx->allocate_temp(DT_UINT8, TensorShape({static_cast<int64_t>(ws_bytes)}), &ws).ok())
+                return FromSdpa(sdpa_hip_fwd_ws(dt, q, k, v, o, stats, ws.flat<uint8>().data(), ws_bytes, B, S_q,
+                                                S_kv, D_qk, D_v, scale, dropout, causal, seed, offset, stream(ctx)));
+        }
         return FromSdpa(sdpa_hip_fwd(dt, q, k, v, o, stats, B, S_q, S_kv, D_qk, D_v, scale, dropout, causal,
                                      seed, offset, stream(ctx)));
     }
