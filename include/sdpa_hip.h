@@ -165,6 +165,14 @@ int sdpa_hip_bwd_dkdv(int dtype, const void* q, const void* k, const void* v, co
 size_t sdpa_hip_bwd_workspace_bytes_ds(int dtype, int B, int S_q, int S_kv, int D_qk, int D_v,
                                        int causal_mask);
 
+/* The largest workspace sdpa_hip_bwd makes use of: that of the dS path, or
+ * for float16 shapes without one whose query side has few tiles (a few
+ * queries against a long memory) the per-row workspace plus the partial dQ
+ * of the workgroups that then share a tile's keys; elsewhere the per-row
+ * workspace.  Any smaller workspace works as described above.               */
+size_t sdpa_hip_bwd_workspace_bytes_full(int dtype, int B, int S_q, int S_kv, int D_qk, int D_v,
+                                         int causal_mask);
+
 /* The three launches of the dS path as separate calls (same arguments as
  * sdpa_hip_bwd; each phase reads what the previous one left in the workspace,
  * in stream order):

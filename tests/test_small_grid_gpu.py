@@ -52,3 +52,35 @@ def test_small_forward(pkg, O, case):
     o_ref, s_ref = O.sdpa_fwd_gate(*make_inputs(c)[:3], **oracle_kw(c))
     for o, s in (outs[0], outs[2]):
         assert maxabs(o, o_ref) <= TOL["f16"]["o"] and maxabs(s, s_ref) <= TOL["f16"]["stats"]
+
+
+BWD = [
+    # dtype, B, S_q, S_kv, D_qk, D_v, causal, dropout; parts of a tile's keys in dQ
+    ("f16", 2, 97, 65, 64, 64, False, 0.1, 1),      # every wave one query block, a one-key tile
+    ("f16", 2, 129, 129, 40, 24, True, 0.1, 1),     # the diagonal blocks, one-row tiles
+    ("f16", 1, 257, 31, 32, 64, False, 0.0, 1),     # one key tile, query blocks more than two rounds
+    ("f16", 3, 33, 1001, 64, 32, False, 0.2, 4),    # dQ in parts, ragged
+    ("f16", 1, 1, 2049, 64, 64, False, 1.5, 8),     # one query; every element dropped
+    ("f16", 2, 160, 160, 128, 128, True, 0.2, 1),   # dS path: sub-tiles that are not stored
+    ("f16", 1, 98, 225, 128, 32, False, 0.1, 1),    # dS path, ragged on both sides
+    ("f16", 1, 129, 70, 24, 72, False, 1.5, 1),     # dS path, every element dropped
+]
+
+
+@pytest.mark.parametrize("case", BWD, ids=["-".join(map(str, c)) for c in BWD])
+def test_small_backward(pkg, O, case):
+    dt, B, S_q, S_kv, D_qk, D_v, causal, p, parts = case
+    c = Cfg("small_bwd", dt, B, S_q, S_kv, D_qk, D_v, causal, p, D_qk ** -0.5, 5, 23)
+    L = pkg.library()
+    dims = (1 if dt == "f16" else 0, B, S_q, S_kv, D_qk, D_v, int(causal))
+    ds, full = L.sdpa_hip_bwd_workspace_bytes_ds(*dims), L.sdpa_hip_bwd_workspace_bytes_full(*dims)
+    assert full == ds + (parts * B * S_q * D_qk * 4 if parts > 1 else 0)
+    run_and_check(pkg, O, c, fp32_sum_allowance=True)
+    # the gradient of another output (o is not this forward's): delta != 0 also where every element is dropped
+    q, k, v, d_o = make_inputs(c)
+    o, s = pkg.sdpa(_t(q), _t(k), _t(v), c.seed, c.offset, dropout=0.0, scale=c.scale, causal_mask=causal)
+    g = pkg.sdpa_grad(_t(q), _t(k), _t(v), o, s, _t(d_o), c.seed, c.offset, dropout=p, scale=c.scale,
+                      causal_mask=causal)
+    ref = O.sdpa_bwd_gate(q, k, v, _np(o), _np(s), d_o, **oracle_kw(c))
+    for a, b in zip(g, ref):
+        assert maxabs(_np(a), b) <= TOL[dt]["grad"] * max(1.0, float(np.abs(b.astype(np.float64)).max()))

@@ -91,6 +91,8 @@ def library():
                                     i32, f32, f32, i32, u64, u64, vp]
     L.sdpa_hip_bwd_workspace_bytes_ds.restype = sz
     L.sdpa_hip_bwd_workspace_bytes_ds.argtypes = [i32] * 7
+    L.sdpa_hip_bwd_workspace_bytes_full.restype = sz
+    L.sdpa_hip_bwd_workspace_bytes_full.argtypes = [i32] * 7
     L.sdpa_hip_bwd_ds_phase.restype = i32
     L.sdpa_hip_bwd_ds_phase.argtypes = [i32, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, i32, i32,
                                         i32, i32, i32, f32, f32, i32, u64, u64, vp]
@@ -208,8 +210,8 @@ def sdpa_grad(q, k, v, o, stats, d_o, seed=0, offset=0, dropout: float = 0.0,
               scale: float = 1.0, causal_mask: bool = False, *, ds_path: bool = True):
     """Gradient op ``SdpaGrad`` (sdpa_ops.cc:34-63): returns ``(dq, dk, dv)``.
 
-    ``ds_path``: give the backward the workspace of its dS path
-    (``sdpa_hip_bwd_workspace_bytes_ds``: float16 or float32 with a feature
+    ``ds_path``: give the backward all the workspace it can use
+    (``sdpa_hip_bwd_workspace_bytes_full``: float16 or float32 with a feature
     size over 64 then stores dS in the dK/dV kernel and forms dQ from it); False gives
     it the per-row workspace only, and both kernels form dS."""
     import torch
@@ -228,8 +230,8 @@ def sdpa_grad(q, k, v, o, stats, d_o, seed=0, offset=0, dropout: float = 0.0,
     dk = torch.empty_like(k)
     dv = torch.empty_like(v)
     if ds_path:
-        ws_bytes = int(L.sdpa_hip_bwd_workspace_bytes_ds(dt, B, S_q, S_kv, D_qk, D_v,
-                                                         int(bool(causal_mask))))
+        ws_bytes = int(L.sdpa_hip_bwd_workspace_bytes_full(dt, B, S_q, S_kv, D_qk, D_v,
+                                                           int(bool(causal_mask))))
     else:
         ws_bytes = int(L.sdpa_hip_bwd_workspace_bytes(B, S_q))
     ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=q.device)

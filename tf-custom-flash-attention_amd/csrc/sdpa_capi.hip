@@ -194,6 +194,15 @@ size_t sdpa_hip_bwd_workspace_bytes_ds(int dtype, int B, int S_q, int S_kv, int 
     return rows + sdpa::DsLayout(S_q, S_kv, causal_mask != 0).bytes(B);
 }
 
+size_t sdpa_hip_bwd_workspace_bytes_full(int dtype, int B, int S_q, int S_kv, int D_qk, int D_v,
+                                         int causal_mask) {
+    const size_t ds = sdpa_hip_bwd_workspace_bytes_ds(dtype, B, S_q, S_kv, D_qk, D_v, causal_mask);
+    if (dtype != SDPA_DTYPE_F16 || B <= 0 || S_q <= 0 || S_kv <= 0 || D_qk <= 0 || D_v < 0) return ds;
+    // the parts of dQ after the row values (shapes without a dS path)
+    const int np = sdpa::dq_parts(sdpa::AttnShape{B, S_q, S_kv, D_qk, D_v}, causal_mask != 0);
+    return np > 1 ? ds + (size_t)np * B * S_q * D_qk * sizeof(float) : ds;
+}
+
 }  // extern "C"
 
 namespace {
@@ -264,6 +273,12 @@ int bwd_entry(Mode mode, int phases, int dtype, const void* q, const void* k, co
         if (e == hipSuccess && (mode == kAuto || mode == kDs2))
             e = f16 ? sdpa::launch_bwd_dq_ds_f16(p, stream) : sdpa::launch_bwd_dq_ds_f32(p, stream);
         return hip_status(e);
+    }
+    p.parts = 1;
+    const size_t full = sdpa_hip_bwd_workspace_bytes_full(dtype, B, S_q, S_kv, D_qk, D_v, causal_mask);
+    if (mode == kAuto && vec && full > rows_bytes && workspace_bytes >= full && aligned16(workspace)) {
+        p.parts = sdpa::dq_parts(p.s, causal_mask != 0);
+        p.part_dq = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + rows_bytes);
     }
     const int ph = mode == kAuto ? (sdpa::kBwdDq | sdpa::kBwdDkDv) : phases;
     if (dtype == SDPA_DTYPE_F16 && vec) return hip_status(sdpa::launch_bwd_f16_dma(p, ph, stream));

@@ -31,6 +31,7 @@
 #include "sdpa_dma.h"
 #include "sdpa_launch.h"
 #include "sdpa_params.h"
+#include "sdpa_parts.h"
 
 namespace sdpa {
 namespace {
@@ -391,6 +392,8 @@ hipError_t launch_bwd_f16_dma(const BwdParams& p, int phases, hipStream_t stream
                     if (err == hipSuccess && (phases & kBwdDkDv) && S_kv > 0) {
                         if constexpr (CK::WAVES == 1 && SDPA_DKDV_SPLIT) {
                             err = launch_bwd_dkdv_f16_split(p, stream);
+                        } else if (dkdv_small(p.s, p.c.causal != 0)) {
+                            err = launch_bwd_dkdv_f16_wave(p, stream);
                         } else {
                             const long long n = (long long)((S_kv + CK::BKV - 1) / CK::BKV) * B;
                             err = launch_kernel<sdpa_bwd_dkdv_f16_dma_kernel<DQK, DV, CA, DR>>(

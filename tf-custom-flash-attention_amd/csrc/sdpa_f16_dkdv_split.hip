@@ -16,6 +16,7 @@
 #include "sdpa_dma.h"
 #include "sdpa_launch.h"
 #include "sdpa_params.h"
+#include "sdpa_parts.h"
 
 // Split-role kernel, who copies the tiles: 0 the dS role; 1 the P role under
 // the causal mask, else the dS role; 2 the P role.
@@ -535,6 +536,7 @@ void sdpa_bwd_dkdv_f16_split_kernel(const BwdParams p, const int win) {
 hipError_t launch_bwd_dkdv_f16_split(const BwdParams& p, hipStream_t stream) {
     const int B = p.s.B, S_kv = p.s.S_kv;
     if (B == 0 || S_kv == 0) return hipSuccess;
+    if (dkdv_small(p.s, p.c.causal != 0)) return launch_bwd_dkdv_f16_wave(p, stream);
     return with_dim(p.s.D_qk, [&](auto dqk) {
         return with_dim(p.s.D_v, [&](auto dv) {
             return with_bool(p.c.causal != 0, [&](auto c) {

@@ -19,6 +19,7 @@
 #include "sdpa_dma.h"
 #include "sdpa_launch.h"
 #include "sdpa_params.h"
+#include "sdpa_parts.h"
 
 namespace sdpa {
 namespace {
@@ -251,6 +252,7 @@ void sdpa_bwd_dq_f16_dma_kernel(const BwdParams p, const int win) {
 hipError_t launch_bwd_dq_f16_dma(const BwdParams& p, hipStream_t stream) {
     const int B = p.s.B, S_q = p.s.S_q;
     if (B == 0 || S_q == 0) return hipSuccess;
+    if (dq_small(p.s, p.c.causal != 0)) return launch_bwd_dq_f16_wave(p, stream);
     return with_dim(p.s.D_qk, [&](auto dqk) {
         return with_dim(p.s.D_v, [&](auto dv) {
             return with_bool(p.c.causal != 0, [&](auto c) {

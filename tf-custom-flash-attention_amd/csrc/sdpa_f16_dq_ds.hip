@@ -21,6 +21,7 @@
 #include "sdpa_dma.h"
 #include "sdpa_launch.h"
 #include "sdpa_params.h"
+#include "sdpa_parts.h"
 
 namespace sdpa {
 namespace {
@@ -257,6 +258,7 @@ hipError_t launch_bwd_dq_ds_f16(const BwdParams& p, hipStream_t stream) {
     const int B = p.s.B, S_q = p.s.S_q;
     if (B == 0 || S_q == 0) return hipSuccess;
     if (!p.ds) return hipErrorInvalidValue;
+    if (dq_ds_small(p.s, p.c.causal != 0)) return launch_bwd_dq_ds_f16_wave(p, stream);
     return with_dim(p.s.D_qk, [&](auto dqk) {
         return with_bool(p.c.causal != 0, [&](auto c) {
             constexpr int DQK = decltype(dqk)::value;

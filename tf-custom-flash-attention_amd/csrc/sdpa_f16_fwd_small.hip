@@ -18,57 +18,23 @@
 // Element semantics are those of sdpa_f16_fwd.hip (hi/lo split of P~
 // included; its test sees the mass of this wave's earlier keys only, which
 // errs towards splitting).
-#include "sdpa_dma.h"
 #include "sdpa_launch.h"
 #include "sdpa_params.h"
 #include "sdpa_parts.h"
+#include "sdpa_wave.h"
 
 namespace sdpa {
 namespace {
 
 constexpr float kTauW = 8.0f;  // lazy-rescale threshold (log2 units), as in sdpa_f16_fwd.hip
 
-// Copies of one 32 x (8 L) fp16 tile by a single wave: copy u fills LDS chunk
-// slots 64 u + lane, i.e. rows 64 u / L + lane / L.  The swizzle repeats every
-// PERIOD copies (TR: the swz_tr layout of tiles read only transposed).
-template <int L, bool TR>
-struct WaveCopy {
-    static constexpr int LOADS = L / 2, RPC = 64 / L;
-    static constexpr int PERIOD = TR || RPC >= 16 ? 1 : 16 / RPC;
-    static constexpr int NV = PERIOD < LOADS ? PERIOD : LOADS;
-    uint32_t voff[NV];
-    __device__ __forceinline__ void init(int lane, int row_bytes, int valid_chunks) {
-#pragma unroll
-        for (int u = 0; u < NV; ++u) {
-            const int r = RPC * u + lane / L;
-            const int c = (lane % L) ^ (TR ? swz_tr<L>(r) : swz<L>(r));
-            voff[u] = c < valid_chunks ? (uint32_t)(r * row_bytes + c * 16) : kOob;
-        }
-    }
-    __device__ __forceinline__ void issue(const RowSrc& src, uint32_t m0) const {
-        const rsrc_t rs = src.at(0);
-#pragma unroll
-        for (int u = 0; u < LOADS; ++u)
-            dma16_at(rs, m0 + 1024u * u, voff[u % NV] + (uint32_t)((u / NV) * NV * RPC * src.row_bytes));
-    }
-};
-
-// s_waitcnt that the compiler does not move LDS reads across: the copies it
-// waits for are invisible to it, and here no barrier follows.
-template <int N>
-__device__ __forceinline__ void wait_copies() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
 template <int DQK, int DV>
 struct FwdWaveCfg {
     static constexpr int NW = 4, NT = 64 * NW, BM = 32, BN = 32;
     static constexpr int LK = DQK / 8, LV = DV / 8;
     static constexpr int KB = BN * DQK * 2, VB = BN * DV * 2, STAGE = KB + VB, RING = 2 * STAGE;
-    // merge area (after the loop): O of every wave with rows of DV + 4
-    // floats (16 bytes apart modulo the banks), then m and l
-    static constexpr int OS = DV + 4, MERGE = NW * BM * OS * 4 + NW * BM * 8;
+    // merge area (after the loop): O of every wave, then m and l
+    static constexpr int OS = acc_stride(DV), MERGE = NW * BM * OS * 4 + NW * BM * 8;
     static constexpr size_t LDS_BYTES = NW * RING > MERGE ? NW * RING : MERGE;
     static_assert(LDS_BYTES <= 160 * 1024, "gfx950 LDS");
     static constexpr int WPE = 2 * LDS_BYTES <= 160 * 1024 ? 2 : 1;
@@ -234,12 +200,7 @@ void sdpa_fwd_f16_wave_kernel(const FwdParams p, const int win) {
         mml[(wave * BM + l32) * 2] = m_run;
         mml[(wave * BM + l32) * 2 + 1] = l_tot;
     }
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<floatx4*>(mo + (wave * BM + l32) * Cfg::OS + 32 * dt + 8 * g + 4 * hh) =
-                (floatx4){oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+    acc_to_lds<DV>(mo, wave * BM + l32, oacc, hh);
     __syncthreads();
     // one thread per four columns of a row
     const bool whole = np == 1;
@@ -268,10 +229,7 @@ void sdpa_fwd_f16_wave_kernel(const FwdParams p, const int win) {
         if (whole) {
             if (c == 0) p.stats[grow] = ((L > 0.f) ? M * kLn2 : kNegInf) + logf(L + kEps);
             const float inv = (L > kEps) ? p.c.keep_scale / L : 0.f;
-            half4 hv;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) hv[e] = (half_t)(acc[e] * inv);
-            *reinterpret_cast<half4*>(static_cast<half_t*>(p.o) + grow * D_v + c) = hv;
+            *reinterpret_cast<half4*>(static_cast<half_t*>(p.o) + grow * D_v + c) = scaled_h4(acc, inv);
         } else {
             const size_t at = (size_t)part * B * S_q + grow;
             if (c == 0) {

@@ -75,6 +75,11 @@ hipError_t launch_bwd_dkdv_f16_split(const BwdParams& p, hipStream_t stream);
 inline bool bwd_ds_shape(int D_qk, int D_v) { return D_qk > 64 || D_v > 64; }
 hipError_t launch_bwd_rows_f16(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dq_ds_f16(const BwdParams& p, hipStream_t stream);
+// The same three kernels, and dQ of the other path, for grids too small to
+// fill the chip (sdpa_f16_bwd_small.hip); p.parts as planned.
+hipError_t launch_bwd_dq_f16_wave(const BwdParams& p, hipStream_t stream);
+hipError_t launch_bwd_dkdv_f16_wave(const BwdParams& p, hipStream_t stream);
+hipError_t launch_bwd_dq_ds_f16_wave(const BwdParams& p, hipStream_t stream);
 // The same path for fp32 (sdpa_f32_dq_ds.hip; its dK/dV phase is launch_bwd
 // with p.ds set, which runs the fp32 split dK/dV kernel storing dS).
 hipError_t launch_bwd_rows_f32(const BwdParams& p, hipStream_t stream);

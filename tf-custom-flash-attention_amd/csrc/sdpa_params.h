@@ -57,6 +57,10 @@ struct BwdParams {
     // dS path only (else null): dS' of every visited (key tile, query block),
     // written by the dK/dV kernel and read by the dQ kernel (DsLayout)
     void* ds;
+    // Small grids (sdpa_parts.h): workgroups that share a query tile's keys in
+    // the dQ kernel, and the workspace of their sums where there are several
+    int parts;
+    float* part_dq;  // [part][B S_q][D_qk]
     AttnShape s;
     AttnScalars c;
 };

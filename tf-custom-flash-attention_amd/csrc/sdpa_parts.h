@@ -6,6 +6,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "sdpa_params.h"
+
 namespace sdpa {
 
 // First of n blocks in part `part` of np (equal lengths, +-1).
@@ -58,6 +60,59 @@ inline FwdPlan fwd_plan(bool f16, int B, int S_q, int S_kv, int D_qk, int D_v, b
     f.o_bytes = (rows * D_v * 4 + 255) & ~(size_t)255;
     f.bytes = f.o_bytes + rows * 8;
     return f;
+}
+
+// ---- backward: where the kernels of sdpa_f16_bwd_small.hip run (times of
+// the whole backward in us, large kernel -> small kernel, dropout 0.1 where
+// S_q = S_kv).  As in the forward a small kernel wins while its workgroups
+// are resident at once, and under the causal mask, where the large kernels
+// wait for their heaviest tiles, up to twice that on long sides.
+inline long long small_tiles(int B, int S, int rows) { return (long long)B * ((S + rows - 1) / rows); }
+
+// dQ at D <= 64, two workgroups per CU.  512 tiles: 36.6 -> 32.4 (B 32, S
+// 512, causal), 61.5 -> 56.5 (B 16, S 1000); 1024 tiles: 37.5 -> 40.6 (B 64,
+// S 512, causal) but 111 -> 103 (B 16, S 2048, causal).
+inline bool dq_small(const AttnShape& s, bool causal) {
+    if (s.D_qk > 64 || s.D_v > 64) return false;
+    return small_tiles(s.B, s.S_q, kSmallRows) <= (causal && s.S_q >= 1000 ? 1024 : 512);
+}
+
+// Workgroups that share a tile's keys in that kernel: as many as give 256
+// workgroups (512 where a dozen blocks would remain per wave), at least two
+// blocks a wave, where it saves each wave at least six blocks (about what the
+// merge kernel costs).  B 16, S_q 64, S_kv 4000: 40.3 in one part, 23.7 in
+// eight; B 64, S_q 64, S_kv 1000: 23.6 in one, 23.9 in two.
+inline int dq_parts(const AttnShape& s, bool causal) {
+    if (causal || !dq_small(s, causal) || s.B <= 0 || s.S_q <= 0) return 1;
+    const long long tiles = small_tiles(s.B, s.S_q, kSmallRows);
+    const long long walk = (small_tiles(1, s.S_kv, kSmallRows) + kSmallWaves - 1) / kSmallWaves;
+    long long n = 256 / tiles;
+    if (n < 1 || walk / n >= 12) n = 512 / tiles;
+    if (n > walk / 2) n = walk / 2;
+    return n < 2 || walk - walk / n < 6 ? 1 : (int)n;
+}
+
+// dK/dV, two workgroups per CU up to D = 64, one at a 128-wide side.  Each of
+// the four waves needs a query block of its own to win.  D = 64: 512 tiles
+// 23.9 -> 19.2 (B 64, S 256, causal), 1024 tiles 25.2 -> 26.3 (B 128, S 256)
+// but 62.1 -> 48.2 (B 32, S 1000, causal), 2048 tiles 66.6 -> 70.3 (B 64).
+// D = 128: 256 tiles 46.8 -> 39.6 (B 16, S 512, causal), 512 tiles 48.2 ->
+// 51.5 (B 32, S 512) but 77.2 -> 69.9 (B 16, S 1000, causal).  S_q 16,
+// S_kv 4000, B 4, D 64: 62.3 -> 64.2.
+inline bool dkdv_small(const AttnShape& s, bool causal) {
+    if (s.S_q <= 3 * kSmallRows) return false;
+    const long long tiles = small_tiles(s.B, s.S_kv, kSmallRows);
+    if (s.D_qk > 64 || s.D_v > 64) return tiles <= (causal && s.S_q >= 1000 ? 512 : 256);
+    return tiles <= (s.S_q >= 512 ? 1024 : 512);
+}
+
+// dQ from the stored dS', 64-query tiles, one workgroup per CU: two rounds of
+// them still win, as the large kernel's tiles are four times as high.  512
+// tiles: 51.7 -> 45.1 (B 64, S 512, D 128, causal), 83.6 -> 77.9 (B 32, S
+// 1000); 1024 tiles: 141 -> 150 (B 64, S 1000) but 161 -> 147 (B 32, S 2048,
+// causal).  B 16, S_q 64, S_kv 4000: 115 -> 56.
+inline bool dq_ds_small(const AttnShape& s, bool causal) {
+    return small_tiles(s.B, s.S_q, 64) <= (causal && s.S_q >= 1000 ? 1024 : 512);
 }
 
 }  // namespace sdpa
