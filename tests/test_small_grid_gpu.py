@@ -54,6 +54,53 @@ def test_small_forward(pkg, O, case):
         assert maxabs(o, o_ref) <= TOL["f16"]["o"] and maxabs(s, s_ref) <= TOL["f16"]["stats"]
 
 
+F32 = [
+    # B, S_q, S_kv, D_qk, D_v, causal, dropout, scale
+    (2, 129, 64, 64, 64, False, 0.1, 0.125),     # one block, a one-row tile
+    (1, 33, 2049, 128, 128, False, 0.0, 0.1),    # 32-key blocks, parts, a one-key tail
+    (2, 65, 65, 37, 5, True, 0.2, -0.2),         # element loads, negated scale
+    (2, 200, 200, 32, 128, True, 0.1, 0.0),      # scale 0
+    (3, 1, 700, 128, 64, False, 1.5, 0.1),       # every element dropped
+]
+
+
+@pytest.mark.parametrize("case", F32, ids=["-".join(map(str, c)) for c in F32])
+def test_f32_forward(pkg, O, case):
+    """The fp32 forward on the bf16 matrix cores: o within 1e-5 and, where
+    keys are divided, the undivided form as well."""
+    B, S_q, S_kv, D_qk, D_v, causal, p, scale = case
+    c = Cfg("f32_fwd", "f32", B, S_q, S_kv, D_qk, D_v, causal, p, scale, 3, 17)
+    q, k, v, _ = make_inputs(c)
+    o_ref, s_ref = O.sdpa_fwd_gate(q, k, v, **oracle_kw(c))
+    L = pkg.library()
+    want = L.sdpa_hip_fwd_workspace_bytes(0, B, S_q, S_kv, D_qk, D_v, int(causal))
+    t = [_t(a) for a in (q, k, v)]
+    for ws_bytes in {want, 0}:
+        ws = torch.empty((max(want, 1),), dtype=torch.uint8, device=t[0].device)
+        o = torch.empty((B, S_q, D_v), dtype=torch.float32, device=t[0].device)
+        s = torch.empty((B, S_q), dtype=torch.float32, device=t[0].device)
+        rc = L.sdpa_hip_fwd_ws(0, *(a.data_ptr() for a in t), o.data_ptr(), s.data_ptr(), ws.data_ptr(), ws_bytes,
+                               B, S_q, S_kv, D_qk, D_v, scale, p, int(causal), c.seed, c.offset,
+                               torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        assert maxabs(_np(o), o_ref) <= TOL["f32"]["o"] and maxabs(_np(s), s_ref) <= TOL["f32"]["stats"]
+
+
+def test_f32_forward_extreme_keys(pkg):
+    """A key of -inf scores weighs 0 (its bf16 parts are NaN past the first),
+    and one near the type's lowest value as well; other rows keep their error."""
+    g = torch.Generator().manual_seed(1)
+    q = (torch.rand((2, 70, 64), generator=g) + 0.1).cuda()
+    k, v = torch.randn((2, 70, 64), generator=g).cuda(), torch.randn((2, 70, 64), generator=g).cuda()
+    q[0] = 1.0
+    k[:, 5] = float("-inf")
+    k[:, 40, 3] = -3.4e38
+    o, _ = pkg.sdpa(q, k, v, scale=0.125)
+    ref = torch.softmax(q.double().cpu() @ k.double().cpu().transpose(1, 2) * 0.125, -1) @ v.double().cpu()
+    assert (o.double().cpu() - ref).abs().max().item() <= 1e-5
+
+
 BWD = [
     # dtype, B, S_q, S_kv, D_qk, D_v, causal, dropout; parts of a tile's keys in dQ
     ("f16", 2, 97, 65, 64, 64, False, 0.1, 1),      # every wave one query block, a one-key tile

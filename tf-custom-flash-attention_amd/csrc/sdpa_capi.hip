@@ -162,7 +162,8 @@ int sdpa_hip_fwd_ws(int dtype, const void* q, const void* k, const void* v, void
     }
     if (dtype == SDPA_DTYPE_F16 && vec)
         return hip_status(plan.small ? sdpa::launch_fwd_f16_wave(p, stream) : sdpa::launch_fwd_f16_dma(p, stream));
-    return hip_status(sdpa::launch_fwd(p, (sdpa::DType)dtype, vec, stream));
+    if (dtype == SDPA_DTYPE_F32) return hip_status(sdpa::launch_fwd_f32(p, vec, stream));
+    return hip_status(sdpa::launch_fwd_f16(p, vec, stream));
 }
 
 size_t sdpa_hip_bwd_workspace_bytes(int B, int S_q) {

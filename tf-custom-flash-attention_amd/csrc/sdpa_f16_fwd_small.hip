@@ -19,6 +19,7 @@
 // included; its test sees the mass of this wave's earlier keys only, which
 // errs towards splitting).
 #include "sdpa_launch.h"
+#include "sdpa_merge.h"
 #include "sdpa_params.h"
 #include "sdpa_parts.h"
 #include "sdpa_wave.h"
@@ -241,56 +242,6 @@ void sdpa_fwd_f16_wave_kernel(const FwdParams p, const int win) {
     }
 }
 
-// Merge of a row's parts: o = sum_i O_i 2^(m_i - M) / l, stats from M and l.
-// One thread per four columns.
-template <typename T>
-__global__ __launch_bounds__(256) void sdpa_fwd_merge_kernel(const FwdParams p) {
-    const int D_v = p.s.D_v, np = p.parts, cpr = (D_v + 3) / 4;
-    const size_t rows = (size_t)p.s.B * p.s.S_q;
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t row = i / cpr;
-    const int c = 4 * (int)(i - row * cpr);
-    if (row >= rows) return;
-    // eight parts at a time: their loads all go out before the first is used
-    // (one part after the other, each waited out the memory latency)
-    constexpr int U = 8;
-    float M = kMaxSentinel, L = 0.f;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < np; k0 += U) {
-        float m[U], l[U], o[U][4];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = k0 + u < np ? k0 + u : np - 1;
-            const size_t at = k * rows + row;
-            m[u] = p.part_ml[2 * at];
-            l[u] = p.part_ml[2 * at + 1];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[u][e] = c + e < D_v ? p.part_o[at * D_v + c + e] : 0.f;
-        }
-        float Mn = M;
-#pragma unroll
-        for (int u = 0; u < U; ++u) Mn = fmaxf(Mn, m[u]);
-        const float a = fast_exp2(M - Mn);
-        L *= a;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] *= a;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const float w = k0 + u < np ? fast_exp2(m[u] - Mn) : 0.f;
-            L = __builtin_fmaf(l[u], w, L);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(o[u][e], w, acc[e]);
-        }
-        M = Mn;
-    }
-    if (c == 0) p.stats[row] = ((L > 0.f) ? M * kLn2 : kNegInf) + logf(L + kEps);
-    const float inv = (L > kEps) ? p.c.keep_scale / L : 0.f;
-    T* o = static_cast<T*>(p.o) + row * D_v + c;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if (c + e < D_v) o[e] = (T)(acc[e] * inv);
-}
-
 }  // namespace
 
 hipError_t launch_fwd_f16_wave(const FwdParams& p, hipStream_t stream) {
@@ -304,14 +255,10 @@ hipError_t launch_fwd_f16_wave(const FwdParams& p, hipStream_t stream) {
                     using Cfg = FwdWaveCfg<DQK, DV>;
                     static_assert(Cfg::BM == kSmallRows && Cfg::BN == kSmallRows && Cfg::NW == kSmallWaves, "planned by fwd_plan");
                     const long long n = (long long)((S_q + Cfg::BM - 1) / Cfg::BM) * p.parts * B;
-                    hipError_t err = launch_kernel<sdpa_fwd_f16_wave_kernel<DQK, DV, decltype(c)::value, decltype(d)::value>>(
+                    const hipError_t err = launch_kernel<sdpa_fwd_f16_wave_kernel<DQK, DV, decltype(c)::value, decltype(d)::value>>(
                         (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p,
                         row_window((size_t)p.s.S_kv * (DQK + DV) * 2));
-                    if (err == hipSuccess && p.parts > 1) {
-                        const long long th = (long long)B * S_q * ((p.s.D_v + 3) / 4);
-                        err = launch_kernel<sdpa_fwd_merge_kernel<half_t>>((unsigned)((th + 255) / 256), 256, 0, stream, p);
-                    }
-                    return err;
+                    return err == hipSuccess && p.parts > 1 ? launch_fwd_merge<half_t>(p, stream) : err;
                 });
             });
         });

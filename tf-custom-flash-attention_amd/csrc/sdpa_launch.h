@@ -50,7 +50,10 @@ hipError_t launch_kernel(unsigned grid, unsigned block, size_t lds, hipStream_t 
     return hipGetLastError();
 }
 
-hipError_t launch_fwd(const FwdParams& p, DType dtype, bool vec, hipStream_t stream);
+// fp16 forward for any D and alignment (sdpa_fwd.hip)
+hipError_t launch_fwd_f16(const FwdParams& p, bool vec, hipStream_t stream);
+// fp32 forward on the bf16 matrix cores (sdpa_f32_fwd.hip)
+hipError_t launch_fwd_f32(const FwdParams& p, bool vec, hipStream_t stream);
 // phases: kBwdDq (dQ kernel, writes delta) and/or kBwdDkDv (reads delta).
 constexpr int kBwdDq = 1, kBwdDkDv = 2;
 hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, int phases, hipStream_t stream);

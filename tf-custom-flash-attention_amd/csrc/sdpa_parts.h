@@ -22,6 +22,40 @@ struct FwdPlan {
     size_t o_bytes, bytes;  // workspace of the parts' O, and in all (0 with one part)
 };
 
+// Parts of the keys of a 128-query tile in the fp32 forward (sdpa_f32_fwd.hip,
+// one workgroup per CU): the number with the least estimated time.  A block
+// (64 keys, 32 where both sides are 128 wide) takes about 0.0215 us per
+// padded feature column of K and V (2.35 measured at 64 + 64, 4.2 at 128 +
+// 64, 2.95 for half a block at 128 + 128), a workgroup about 4 us besides,
+// and the merge about 4 us and its traffic at 3 TB/s.  Under the causal mask
+// a tile has half of the blocks on average, the last one all of them.
+// Undivided -> chosen, us: B 8, S_q 1, S_kv 8000, D 64: 288 -> 22.6 (32
+// parts); B 64, S_q 64, S_kv 2000, D 128: 194 -> 65 (4); B 24, S 700, D 64:
+// 38 -> 38 (1; in two parts 57: a second round of workgroups).
+inline long long fwd_f32_parts(int B, int S_q, int S_kv, int pq, int pv, int D_v, bool causal) {
+    const bool wide = pq == 128 && pv == 128;
+    const long long tiles = (long long)B * ((S_q + 127) / 128);
+    const long long blocks = ((long long)S_kv + (wide ? 31 : 63)) / (wide ? 32 : 64);
+    if (tiles > 256 || blocks < 2) return 1;
+    const double t = wide ? 2.95 : 0.0215 * (pq + pv);
+    long long best = 1;
+    double best_us = 0;
+    for (long long n = 1; n <= blocks && n <= 64; ++n) {
+        const double chain = 4 + (double)((blocks + n - 1) / n) * t;
+        double us = (double)((tiles * n + 255) / 256) * chain;
+        if (causal) {
+            const double work = (double)tiles * (4 * n + 0.5 * blocks * t) / 256 + chain / 2;
+            us = work > chain ? work : chain;
+        }
+        if (n > 1) us += 4 + (double)n * B * S_q * D_v * 8 / 3e6;
+        if (n == 1 || us < 0.95 * best_us) {
+            best = n;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
 // The fp16 forward of a shape, from its count of 32-query tiles (all times
 // in us, 128-query kernel -> 32-query kernel).
 //
@@ -43,8 +77,19 @@ struct FwdPlan {
 // B 128, S_q 1, S_kv 1000, D 128: 14.5 in one, 18.7 in two.
 inline FwdPlan fwd_plan(bool f16, int B, int S_q, int S_kv, int D_qk, int D_v, bool causal) {
     FwdPlan f{false, 1, 0, 0};
-    if (!f16 || B <= 0 || S_q <= 0) return f;
+    if (B <= 0 || S_q <= 0) return f;
     const auto pad = [](int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); };
+    const auto divide = [&](long long n) {
+        f.parts = (int)n;
+        const size_t rows = (size_t)f.parts * B * S_q;
+        f.o_bytes = (rows * D_v * 4 + 255) & ~(size_t)255;
+        f.bytes = f.o_bytes + rows * 8;
+    };
+    if (!f16) {
+        divide(fwd_f32_parts(B, S_q, S_kv, pad(D_qk), pad(D_v), D_v, causal));
+        if (f.parts == 1) f.o_bytes = f.bytes = 0;
+        return f;
+    }
     const long long tiles = (long long)B * ((S_q + kSmallRows - 1) / kSmallRows);
     const long long slots = pad(D_qk) + pad(D_v) <= 160 ? 512 : 256;
     f.small = tiles <= (causal && S_q >= 1000 ? 2 * slots : slots);
@@ -55,10 +100,7 @@ inline FwdPlan fwd_plan(bool f16, int B, int S_q, int S_kv, int D_qk, int D_v, b
     if (slots == 512 && (n < 1 || walk / n >= 12)) n = slots / tiles;
     if (n > walk / 2) n = walk / 2;
     if (n < 2 || walk - walk / n < 9) return f;
-    f.parts = (int)n;
-    const size_t rows = (size_t)f.parts * B * S_q;
-    f.o_bytes = (rows * D_v * 4 + 255) & ~(size_t)255;
-    f.bytes = f.o_bytes + rows * 8;
+    divide(n);
     return f;
 }
 
