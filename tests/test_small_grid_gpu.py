@@ -111,6 +111,10 @@ BWD = [
     ("f16", 2, 160, 160, 128, 128, True, 0.2, 1),   # dS path: sub-tiles that are not stored
     ("f16", 1, 98, 225, 128, 32, False, 0.1, 1),    # dS path, ragged on both sides
     ("f16", 1, 129, 70, 24, 72, False, 1.5, 1),     # dS path, every element dropped
+    ("f32", 2, 33, 129, 64, 64, False, 0.1, 1),     # a one-row query block, a one-key tile
+    ("f32", 1, 65, 65, 37, 5, True, 0.1, 1),        # element loads, the diagonal
+    ("f32", 2, 160, 160, 128, 128, True, 0.2, 1),   # dS path
+    ("f32", 1, 31, 257, 128, 32, False, 1.5, 1),    # dS path, every element dropped
 ]
 
 

@@ -252,6 +252,7 @@ int bwd_entry(Mode mode, int phases, int dtype, const void* q, const void* k, co
     p.stats2 = static_cast<float*>(workspace);
     p.delta = static_cast<float*>(workspace) + (size_t)B * S_q;
     p.ds = nullptr;
+    p.parts = p.kv_parts = 1;
     p.s = sdpa::AttnShape{B, S_q, S_kv, D_qk, D_v};
     p.c = make_scalars(scale, dropout, causal_mask, seed, offset, true);
     const bool vec = vec_ok(dtype, D_qk, D_v,
@@ -270,12 +271,11 @@ int bwd_entry(Mode mode, int phases, int dtype, const void* q, const void* k, co
             e = f16 ? sdpa::launch_bwd_rows_f16(p, stream) : sdpa::launch_bwd_rows_f32(p, stream);
         if (e == hipSuccess && (mode == kAuto || mode == kDs1))
             e = f16 ? sdpa::launch_bwd_dkdv_f16_split(p, stream)
-                    : sdpa::launch_bwd(p, sdpa::DType::F32, true, sdpa::kBwdDkDv, stream);
+                    : sdpa::launch_bwd_dkdv_f32(p, true, stream);
         if (e == hipSuccess && (mode == kAuto || mode == kDs2))
             e = f16 ? sdpa::launch_bwd_dq_ds_f16(p, stream) : sdpa::launch_bwd_dq_ds_f32(p, stream);
         return hip_status(e);
     }
-    p.parts = 1;
     const size_t full = sdpa_hip_bwd_workspace_bytes_full(dtype, B, S_q, S_kv, D_qk, D_v, causal_mask);
     if (mode == kAuto && vec && full > rows_bytes && workspace_bytes >= full && aligned16(workspace)) {
         p.parts = sdpa::dq_parts(p.s, causal_mask != 0);

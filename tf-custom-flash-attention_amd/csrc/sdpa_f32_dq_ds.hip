@@ -1,11 +1,11 @@
 // sdpa_f32_dq_ds.hip -- the dS path of the fp32 SdpaGrad for gfx950: dQ as a
-// product with the dS the fp32 split dK/dV kernel stored (DsLayout32), instead
+// product with the dS the fp32 dK/dV kernel stored (DsLayout32), instead
 // of the dQ kernel that forms S, P, dP and dS once more (sdpa_bwd.hip).
 //
 // Order of the path (sdpa_capi.hip):
 //   1. row kernel  -- delta (and stats2) per query row into the workspace, as
 //                     the other path's dQ kernel writes them first;
-//   2. dK/dV       -- sdpa_bwd_dkdv_f32_split_kernel with p.ds set: its dS
+//   2. dK/dV       -- sdpa_f32_dkdv.hip with p.ds set: its dS
 //                     role stores every dS it forms;
 //   3. dQ          -- dQ^T = K^T dS^T per 32 queries, scaled once at the store.
 // In fp32 the products run on v_mfma_f32_32x32x2_f32, so dQ stays bound by

@@ -83,8 +83,10 @@ hipError_t launch_bwd_dq_ds_f16(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dq_f16_wave(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dkdv_f16_wave(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dq_ds_f16_wave(const BwdParams& p, hipStream_t stream);
-// The same path for fp32 (sdpa_f32_dq_ds.hip; its dK/dV phase is launch_bwd
-// with p.ds set, which runs the fp32 split dK/dV kernel storing dS).
+// The same path for fp32 (sdpa_f32_dq_ds.hip, sdpa_f32_dkdv.hip).
+// fp32 dK/dV on the bf16 matrix cores (sdpa_f32_dkdv.hip); with p.ds set it
+// also stores dS
+hipError_t launch_bwd_dkdv_f32(const BwdParams& p, bool vec, hipStream_t stream);
 hipError_t launch_bwd_rows_f32(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dq_ds_f32(const BwdParams& p, hipStream_t stream);
 

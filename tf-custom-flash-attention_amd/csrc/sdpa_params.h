@@ -61,6 +61,10 @@ struct BwdParams {
     // the dQ kernel, and the workspace of their sums where there are several
     int parts;
     float* part_dq;  // [part][B S_q][D_qk]
+    // fp32 kernels: workgroups that share a key tile's query blocks
+    int kv_parts;
+    float* part_dk;  // [part][B S_kv][D_qk]
+    float* part_dv;  // [part][B S_kv][D_v]
     AttnShape s;
     AttnScalars c;
 };
