@@ -684,11 +684,17 @@ hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, int phases, hip
                         if (err == hipSuccess && (phases & kBwdDkDv))
                             err = launch_kernel<sdpa_bwd_dkdv_f16_kernel<DQK, DV, V, D>>(gk, CK::NT, CK::LDS_BYTES, stream, p);
                     } else {
-                        using CQ = BwdQF32Cfg<DQK, DV>;
-                        const unsigned gq = (unsigned)(((S_q + CQ::BM - 1) / CQ::BM) * B);
-                        if (phases & kBwdDq)
-                            err = launch_kernel<sdpa_bwd_dq_f32_kernel<DQK, DV, V, D>>(gq, CQ::NT, CQ::LDS_BYTES, stream, p);
+                        if (phases & kBwdDq) {
+                            if constexpr (DQK == 128 || DV == 128) {
+                                using CQ = BwdQF32Cfg<DQK, DV>;
+                                const unsigned gq = (unsigned)(((S_q + CQ::BM - 1) / CQ::BM) * B);
+                                err = launch_kernel<sdpa_bwd_dq_f32_kernel<DQK, DV, V, D>>(gq, CQ::NT, CQ::LDS_BYTES, stream, p);
+                            } else {
+                                err = launch_bwd_dq_f32(p, V, stream);
+                            }
+                        }
                         if (err == hipSuccess && (phases & kBwdDkDv)) err = launch_bwd_dkdv_f32(p, V, stream);
+                        if (err == hipSuccess) err = launch_bwd_merge_f32(p, stream);
                     }
                     return err;
                 });

@@ -198,10 +198,11 @@ size_t sdpa_hip_bwd_workspace_bytes_ds(int dtype, int B, int S_q, int S_kv, int 
 size_t sdpa_hip_bwd_workspace_bytes_full(int dtype, int B, int S_q, int S_kv, int D_qk, int D_v,
                                          int causal_mask) {
     const size_t ds = sdpa_hip_bwd_workspace_bytes_ds(dtype, B, S_q, S_kv, D_qk, D_v, causal_mask);
-    if (dtype != SDPA_DTYPE_F16 || B <= 0 || S_q <= 0 || S_kv <= 0 || D_qk <= 0 || D_v < 0) return ds;
-    // the parts of dQ after the row values (shapes without a dS path)
-    const int np = sdpa::dq_parts(sdpa::AttnShape{B, S_q, S_kv, D_qk, D_v}, causal_mask != 0);
-    return np > 1 ? ds + (size_t)np * B * S_q * D_qk * sizeof(float) : ds;
+    if ((dtype != SDPA_DTYPE_F16 && dtype != SDPA_DTYPE_F32) || B <= 0 || S_q <= 0 || S_kv <= 0 || D_qk <= 0 || D_v < 0)
+        return ds;
+    // behind the row values (shapes without a dS path)
+    return ds + sdpa::bwd_parts(dtype == SDPA_DTYPE_F16, sdpa::AttnShape{B, S_q, S_kv, D_qk, D_v}, causal_mask != 0).floats() *
+                    sizeof(float);
 }
 
 }  // extern "C"
@@ -276,10 +277,15 @@ int bwd_entry(Mode mode, int phases, int dtype, const void* q, const void* k, co
             e = f16 ? sdpa::launch_bwd_dq_ds_f16(p, stream) : sdpa::launch_bwd_dq_ds_f32(p, stream);
         return hip_status(e);
     }
-    const size_t full = sdpa_hip_bwd_workspace_bytes_full(dtype, B, S_q, S_kv, D_qk, D_v, causal_mask);
-    if (mode == kAuto && vec && full > rows_bytes && workspace_bytes >= full && aligned16(workspace)) {
-        p.parts = sdpa::dq_parts(p.s, causal_mask != 0);
+    // the parts' sums behind the row values
+    const sdpa::BwdParts parts = sdpa::bwd_parts(dtype == SDPA_DTYPE_F16, p.s, causal_mask != 0);
+    if (mode == kAuto && (vec || dtype == SDPA_DTYPE_F32) && parts.floats() > 0 && aligned16(workspace) &&
+        workspace_bytes >= rows_bytes + parts.floats() * sizeof(float)) {
+        p.parts = parts.q;
+        p.kv_parts = parts.kv;
         p.part_dq = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + rows_bytes);
+        p.part_dk = p.part_dq + parts.dq_floats;
+        p.part_dv = p.part_dk + parts.dk_floats;
     }
     const int ph = mode == kAuto ? (sdpa::kBwdDq | sdpa::kBwdDkDv) : phases;
     if (dtype == SDPA_DTYPE_F16 && vec) return hip_status(sdpa::launch_bwd_f16_dma(p, ph, stream));

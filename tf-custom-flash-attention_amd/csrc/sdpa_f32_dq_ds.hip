@@ -8,15 +8,13 @@
 //   2. dK/dV       -- sdpa_f32_dkdv.hip with p.ds set: its dS
 //                     role stores every dS it forms;
 //   3. dQ          -- dQ^T = K^T dS^T per 32 queries, scaled once at the store.
-// In fp32 the products run on v_mfma_f32_32x32x2_f32, so dQ stays bound by
-// its one product (the recomputing kernel executes three).
 //
 // Element semantics (sdpa/sdpa_bwd.cu.cc:291-327): dQ_i = scale sum_j dS_ij
 // K_j with dS as the dK/dV kernel forms it (P gated at 1e-6, the dropout
 // decision, dP scaled by 1/(1-p) for kept elements).
 #include <type_traits>
 
-#include "sdpa_dma.h"
+#include "sdpa_bf3.h"
 #include "sdpa_launch.h"
 #include "sdpa_params.h"
 
@@ -57,146 +55,123 @@ __global__ __launch_bounds__(256) void sdpa_bwd_rows_f32_kernel(const BwdParams 
 }
 
 // ---------------------------------------------------------------------------
-// dQ from the stored dS.  Four waves of 32 queries (128 per workgroup): a
-// wave owns one stored query block.  Key steps of 32 (one stored key group)
-// through two LDS stages of the K tile (32 rows of D_qk floats, row-major)
-// and each wave's dS tile (one stored 4 KB key group, copied as it lies).  Each
-// v_mfma_f32_32x32x2_f32 takes a key pair: lane (l32, hh) reads
-// K[2 p + hh][32 dt + l32] (the A operand K^T) and dS[2 p + hh][l32] (the B
-// operand dS^T, lane = query position), so the accumulators hold dQ^T with
-// lane = query position, and lane l32 stores query pi(l32) of the block.
+// dQ from the stored dS, on the bf16 matrix cores (sdpa_bf3.h).  128 queries
+// per workgroup, a stored query block of 32 for each group of waves; the two
+// waves of a group, on one SIMD, share its keys (one stored key group of 32
+// per 64-key step each; their sums are added through LDS at the end).  The K
+// tile is staged through registers and cut into its parts on the way; each
+// wave's 4 KB dS tile is copied as it lies, read per key as stored (lane =
+// query position) and cut in registers.  Lane l32 stores query pi(l32).
+//
+// B 64, S_q 512, S_kv 16384, D_qk 128 (2.1 GB of dS): 1.08 ms on
+// v_mfma_f32_32x32x2_f32 (81% busy), DQDS_MS here.
 // ---------------------------------------------------------------------------
 template <int DQK>
 struct DqDs32Cfg {
-    static constexpr int NW = 4, NT = 64 * NW, BM = 32 * NW, BN = 32, NSTAGE = 2;
-    static constexpr int LK = DQK / 4;           // 16-byte chunks per K row
-    static constexpr int KB = BN * DQK * 4;      // K tile
-    static constexpr int SB = BN * 32 * 4;       // one wave's dS tile (4 KB)
-    static constexpr int CPW = KB / 1024 / NW;   // K copies of 1 KB per wave
-    static constexpr int STAGE = KB + NW * SB;
-    static constexpr size_t LDS_BYTES = NSTAGE * (size_t)STAGE;
-    static_assert(CPW >= 1 && KB % (1024 * NW) == 0, "every wave copies whole KB of the K tile");
-    static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per CU");
+    static constexpr int NT = 512, BM = 128, BN = 64;
+    using KT = Bf3Tile<BN, DQK / 8>;
+    static constexpr int SB = 4096;  // one wave's dS tile
+    static constexpr int SOFF = 2 * KT::BYTES;
+    static constexpr int OS = DQK + 4, MERGE = BM * OS * 4;  // after the loop
+    static constexpr size_t LDS_BYTES = SOFF + 16 * SB > MERGE ? SOFF + 16 * SB : MERGE;
+    static_assert(LDS_BYTES <= 160 * 1024, "gfx950 LDS");
 };
 
 template <int DQK, bool CAUSAL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void sdpa_bwd_dq_ds_f32_kernel(const BwdParams p, const int win) {
     using Cfg = DqDs32Cfg<DQK>;
-    constexpr int BM = Cfg::BM, BN = Cfg::BN, LK = Cfg::LK, NSTAGE = Cfg::NSTAGE, CPW = Cfg::CPW;
-    constexpr int NDT = DQK / 32;
-    static_assert(DsLayout32::KT % BN == 0 && BN == DsLayout32::QBK, "steps tile the stored key groups");
-    static_assert(NSTAGE == 2, "one step of copies ahead");
+    using KT = typename Cfg::KT;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, LK = DQK / 8, NDT = DQK / 32;
+    static_assert(DsLayout32::KT % BN == 0 && DsLayout32::QBK == 32, "steps tile the stored key groups");
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wq = wave & 3, wk = wave >> 2;
     const int B = p.s.B, S_q = p.s.S_q, S_kv = p.s.S_kv, D_qk = p.s.D_qk;
     const int tiles = (S_q + BM - 1) / BM;
     int b, qt;
     xcd_map(blockIdx.x, B * tiles, tiles, CAUSAL, win, b, qt);
-    const int qw0 = qt * BM + 32 * wave, qb = qw0 / DsLayout32::QBK;
+    const int qw0 = qt * BM + 32 * wq, qb = qw0 / DsLayout32::QBK;
     const int pq = 8 * ((l32 >> 2) & 3) + 4 * (l32 >> 4) + (l32 & 3);  // stored position -> query
     const DsLayout32 dsl(S_q, S_kv, CAUSAL);
     const unsigned char* dsb = static_cast<const unsigned char*>(p.ds);
+    const float* Kb = static_cast<const float*>(p.k) + (size_t)b * S_kv * D_qk;
+    const int nsteps = ((CAUSAL ? min(S_kv, qt * BM + BM) : S_kv) + BN - 1) / BN;
 
     // The dK/dV kernel stored this wave's block at the key group kv0 under
     // the same predicate (its `live`).
     auto live = [&](int kv0) { return qw0 < S_q && kv0 < S_kv && !(CAUSAL && qw0 + 31 < kv0); };
-
-    // K tile copies: copy u of wave w fills LDS bytes (CPW w + u) KB + 16
-    // lane, i.e. chunk slot s = 64 (CPW w + u) + lane: row s / LK, slot
-    // s % LK.  Odd rows hold chunk slot ^ 8 (D_qk >= 64), so the two rows of
-    // a key pair, 256 or 512 bytes apart, fall in different bank halves.
-    constexpr int SWZ = DQK >= 64 ? 8 : 0;
-    const RowSrc ksrc = row_src(p.k, (size_t)b * S_kv, S_kv, D_qk * 4);
-    uint32_t kvoff[CPW];
+    const uint32_t s0 = (uint32_t)(Cfg::SOFF + 2 * Cfg::SB * wave);  // this wave's two dS stages
+    auto copy_ds = [&](int step) {
+        const int kv0 = step * BN + 32 * wk;
+        if (!live(kv0)) return;
+        const unsigned char* src = dsb + dsl.offset(b, kv0 / DsLayout32::KT, qb) + ((kv0 % DsLayout32::KT) / 32) * 4096;
+        const rsrc_t rs = make_rsrc(uniform_ptr(src), Cfg::SB);
+        const uint32_t m0 = lds_base() + s0 + (uint32_t)((step & 1) * Cfg::SB);
+        // dS is read once: non-temporal
 #pragma unroll
-    for (int u = 0; u < CPW; ++u) {
-        const int s = 64 * (CPW * wave + u) + lane, r = s / LK;
-        const int c = (s % LK) ^ ((r & 1) ? SWZ : 0);
-        kvoff[u] = c < D_qk / 4 ? (uint32_t)(r * D_qk * 4 + c * 16) : kOob;
-    }
-    const uint32_t lds0 = lds_base();
-    const int kv_end = CAUSAL ? min(S_kv, qt * BM + BM) : S_kv;
-    const int nsteps = (kv_end + BN - 1) / BN;
-    // copies of step `step` into stage step % 2: the wave's share of the K
-    // tile and, when its block is live there, its dS tile (4 KB)
-    auto issue = [&](int step) {
-        const int kv0 = step * BN;
-        const uint32_t so = (uint32_t)((step % NSTAGE) * Cfg::STAGE);
-        const rsrc_t rk = ksrc.shifted(kv0).at(0);
-#pragma unroll
-        for (int u = 0; u < CPW; ++u) dma16_at(rk, lds0 + so + 1024u * (uint32_t)(CPW * wave + u), kvoff[u]);
-        if (live(kv0)) {
-            const unsigned char* src =
-                dsb + dsl.offset(b, kv0 / DsLayout32::KT, qb) + ((kv0 % DsLayout32::KT) / 32) * 4096;
-            // dS is read once: non-temporal
-            const rsrc_t rs = RowSrc{uniform_ptr(src), 32, 128, 0x7FFFFFFF / 128}.at(0);
-            const uint32_t m0 = lds0 + so + (uint32_t)(Cfg::KB + Cfg::SB * wave);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) dma16_at_nt(rs, m0 + 1024u * u, (uint32_t)(16 * lane + 1024 * u));
-        }
+        for (int u = 0; u < 4; ++u) dma16_at_nt(rs, m0 + 1024u * u, (uint32_t)(16 * lane + 1024 * u));
     };
+    Bf3Stage<BN, DQK, Cfg::NT, true> kst;
+    auto load_k = [&](int step) { kst.load(Kb, step * BN, S_kv - step * BN, D_qk, D_qk, tid); };
+    auto store_k = [&](int step) { kst.store(smem + (step & 1) * KT::BYTES, tid); };
 
+    SwzLane<LK> swK;
+    swK.init(lane);
+    // dS of key r, position l32 sits at slot32(r, l32) = base + 16 (r ^ (u + 4
+    // h)); for the keys 8 i + 4 hh + e of an operand the XOR term stays below
+    // 8: one lane base per e, 128 i as an immediate
+    int sbase[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sbase[e] = DsLayout32::slot32(4 * hh + e, l32);
     floatx16 acc[NDT];
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) acc[dt] = floatx16{};
-    // lane terms of the reads: K[2 p + hh][32 dt + l32] and dS[2 p + hh][l32].
-    // dS sits at DsLayout32::slot32(2 p + hh, l32), with u = (l32 >> 2) & 3
-    // and h = l32 >> 4 from the lane's query position; for p = 4 i + j its
-    // key slot is 8 i + ((2 j + hh) ^ (u + 4 h)) (the XOR term stays below 8),
-    // so one lane base per j and the immediate 128 i.
-    const int krow_sw = hh ? SWZ : 0;
-    int sbase[4];
+
+    if (nsteps > 0) {
+        copy_ds(0);
+        load_k(0);
+        store_k(0);
+        wait_vm();
+        if (nsteps > 1) load_k(1);
+    }
+    __syncthreads();
+    for (int step = 0; step < nsteps; ++step) {
+        // the other stages were released at the last barrier
+        if (step + 1 < nsteps) copy_ds(step + 1);
+        if (live(step * BN + 32 * wk)) {
+            const uint32_t ks0 = (uint32_t)((step & 1) * KT::BYTES);
+            const unsigned char* Ss = smem + s0 + (step & 1) * Cfg::SB;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sbase[j] = DsLayout32::slot32(2 * j + hh, l32);
-    // All of a step's operands are read first (BN / 2 (1 + NDT) floats per
-    // lane), so that each MFMA finds its operands landed instead of waiting
-    // out the LDS latency of a read issued just before it.
-    auto step_mfma = [&](uint32_t so) {
-        const float* Ks = reinterpret_cast<const float*>(smem + so);
-        const unsigned char* Ss = smem + so + Cfg::KB + Cfg::SB * wave;
-        float bv[BN / 2], av[BN / 2][NDT];
+            for (int j = 0; j < 2; ++j) {
+                const Bf3 ds = cut8([&](int i) {
+                    return *reinterpret_cast<const float*>(Ss + sbase[i & 3] + 128 * (2 * j + (i >> 2)));
+                });
 #pragma unroll
-        for (int pr = 0; pr < BN / 2; ++pr) {
-            const int r = 2 * pr + hh;
-            bv[pr] = *reinterpret_cast<const float*>(Ss + sbase[pr & 3] + 128 * (pr >> 2));
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) {
-                const int c = (8 * dt + (l32 >> 2)) ^ krow_sw;
-                av[pr][dt] = Ks[r * DQK + 4 * c + (l32 & 3)];
+                for (int dt = 0; dt < NDT; ++dt)
+                    acc[dt] = mfma_bf3(KT::tr(ks0 + swK.tr0, ks0 + swK.tr1, dt, 32 * wk + 16 * j), ds, acc[dt]);
             }
         }
-#pragma unroll
-        for (int pr = 0; pr < BN / 2; ++pr)
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) acc[dt] = mfma_f32(av[pr][dt], bv[pr], acc[dt]);
-    };
-
-    if (nsteps > 0) issue(0);
-    for (int step = 0; step < nsteps; ++step) {
-        wait_vm();
+        if (step + 1 < nsteps) store_k(step + 1);
+        wait_vm();  // the next step's dS
+        if (step + 2 < nsteps) load_k(step + 2);
         __syncthreads();
-        // stage (step + 1) % 2 held step - 1, which every wave has finished
-        if (step + 1 < nsteps) issue(step + 1);
-        if (live(step * BN)) step_mfma((uint32_t)((step % NSTAGE) * Cfg::STAGE));
     }
 
+    float* m = reinterpret_cast<float*>(smem) + (32 * wq + l32) * Cfg::OS;
+    if (wk == 1) store_rows_f32<DQK, true>(m, acc, 1.f, hh, DQK);
+    __syncthreads();
     const int my_q = qw0 + pq;
-    if (my_q < S_q) {
-        const float f = p.c.scale;
-        float* dQb = static_cast<float*>(p.dq) + ((size_t)b * S_q + my_q) * D_qk;
+    if (wk == 1 || my_q >= S_q) return;
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
+    for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const int d0 = 32 * dt + 8 * g4 + 4 * hh;
-                floatx4 fv;
+        for (int g = 0; g < 4; ++g) {
+            const floatx4 x = *reinterpret_cast<const floatx4*>(m + 32 * dt + 8 * g + 4 * hh);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) fv[e] = acc[dt][4 * g4 + e] * f;
-                if (d0 < D_qk) *reinterpret_cast<floatx4*>(dQb + d0) = fv;
-            }
-    }
+            for (int e = 0; e < 4; ++e) acc[dt][4 * g + e] += x[e];
+        }
+    store_rows_f32<DQK, true>(static_cast<float*>(p.dq) + ((size_t)b * S_q + my_q) * D_qk, acc, p.c.scale, hh, D_qk);
 }
 
 }  // namespace

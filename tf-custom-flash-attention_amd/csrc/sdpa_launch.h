@@ -84,6 +84,11 @@ hipError_t launch_bwd_dq_f16_wave(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dkdv_f16_wave(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dq_ds_f16_wave(const BwdParams& p, hipStream_t stream);
 // The same path for fp32 (sdpa_f32_dq_ds.hip, sdpa_f32_dkdv.hip).
+// fp32 dQ of the path without stored dS at D <= 64, on the bf16 matrix cores,
+// and the sums of the parts where p.parts or p.kv_parts are more than one
+// (sdpa_f32_dq.hip)
+hipError_t launch_bwd_dq_f32(const BwdParams& p, bool vec, hipStream_t stream);
+hipError_t launch_bwd_merge_f32(const BwdParams& p, hipStream_t stream);
 // fp32 dK/dV on the bf16 matrix cores (sdpa_f32_dkdv.hip); with p.ds set it
 // also stores dS
 hipError_t launch_bwd_dkdv_f32(const BwdParams& p, bool vec, hipStream_t stream);

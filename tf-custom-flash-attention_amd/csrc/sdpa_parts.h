@@ -22,38 +22,46 @@ struct FwdPlan {
     size_t o_bytes, bytes;  // workspace of the parts' O, and in all (0 with one part)
 };
 
-// Parts of the keys of a 128-query tile in the fp32 forward (sdpa_f32_fwd.hip,
-// one workgroup per CU): the number with the least estimated time.  A block
-// (64 keys, 32 where both sides are 128 wide) takes about 0.0215 us per
-// padded feature column of K and V (2.35 measured at 64 + 64, 4.2 at 128 +
-// 64, 2.95 for half a block at 128 + 128), a workgroup about 4 us besides,
-// and the merge about 4 us and its traffic at 3 TB/s.  Under the causal mask
-// a tile has half of the blocks on average, the last one all of them.
-// Undivided -> chosen, us: B 8, S_q 1, S_kv 8000, D 64: 288 -> 22.6 (32
-// parts); B 64, S_q 64, S_kv 2000, D 128: 194 -> 65 (4); B 24, S 700, D 64:
-// 38 -> 38 (1; in two parts 57: a second round of workgroups).
-inline long long fwd_f32_parts(int B, int S_q, int S_kv, int pq, int pv, int D_v, bool causal) {
-    const bool wide = pq == 128 && pv == 128;
-    const long long tiles = (long long)B * ((S_q + 127) / 128);
-    const long long blocks = ((long long)S_kv + (wide ? 31 : 63)) / (wide ? 32 : 64);
+// The number of parts with the least estimated time for `tiles` tiles of
+// `blocks` streamed blocks each on 256 workgroups at a time (one per CU):
+// block_us per block, 4 us per workgroup besides, and with several parts the
+// second kernel, merge_us and its traffic (part_bytes per part, written and
+// read, at 2.5 TB/s).  Under the causal mask a tile has half of the blocks
+// on average, one of them all.
+inline int least_time_parts(long long tiles, long long blocks, bool causal, double block_us, double merge_us,
+                            double part_bytes) {
     if (tiles > 256 || blocks < 2) return 1;
-    const double t = wide ? 2.95 : 0.0215 * (pq + pv);
-    long long best = 1;
+    int best = 1;
     double best_us = 0;
-    for (long long n = 1; n <= blocks && n <= 64; ++n) {
-        const double chain = 4 + (double)((blocks + n - 1) / n) * t;
+    for (int n = 1; n <= blocks && n <= 64; ++n) {
+        const double chain = 4 + (double)((blocks + n - 1) / n) * block_us;
         double us = (double)((tiles * n + 255) / 256) * chain;
         if (causal) {
-            const double work = (double)tiles * (4 * n + 0.5 * blocks * t) / 256 + chain / 2;
+            const double work = (double)tiles * (4 * n + 0.5 * blocks * block_us) / 256 + chain / 2;
             us = work > chain ? work : chain;
         }
-        if (n > 1) us += 4 + (double)n * B * S_q * D_v * 8 / 3e6;
+        if (n > 1) us += merge_us + n * part_bytes / 2.5e6;
         if (n == 1 || us < 0.95 * best_us) {
             best = n;
             best_us = us;
         }
     }
     return best;
+}
+
+inline int pad_dim(int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }
+
+// Parts of the keys of a 128-query tile in the fp32 forward (sdpa_f32_fwd.hip).
+// A block (64 keys, 32 where both sides are 128 wide) takes about 0.0215 us
+// per padded feature column of K and V: 2.35 measured at 64 + 64, 4.2 at 128
+// + 64, 2.95 for 32 keys at 128 + 128.  Undivided -> chosen, us: B 8, S_q 1,
+// S_kv 8000, D 64: 288 -> 22.6 (32 parts); B 64, S_q 64, S_kv 2000, D 128:
+// 194 -> 65 (4); B 24, S 700, D 64: 38 (1; in two parts 57: a second round).
+inline int fwd_f32_parts(int B, int S_q, int S_kv, int D_qk, int D_v, bool causal) {
+    const int pq = pad_dim(D_qk), pv = pad_dim(D_v);
+    const bool wide = pq == 128 && pv == 128;
+    return least_time_parts((long long)B * ((S_q + 127) / 128), ((long long)S_kv + (wide ? 31 : 63)) / (wide ? 32 : 64),
+                            causal, wide ? 2.95 : 0.0215 * (pq + pv), 4, 8.0 * B * S_q * D_v);
 }
 
 // The fp16 forward of a shape, from its count of 32-query tiles (all times
@@ -78,7 +86,6 @@ inline long long fwd_f32_parts(int B, int S_q, int S_kv, int pq, int pv, int D_v
 inline FwdPlan fwd_plan(bool f16, int B, int S_q, int S_kv, int D_qk, int D_v, bool causal) {
     FwdPlan f{false, 1, 0, 0};
     if (B <= 0 || S_q <= 0) return f;
-    const auto pad = [](int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); };
     const auto divide = [&](long long n) {
         f.parts = (int)n;
         const size_t rows = (size_t)f.parts * B * S_q;
@@ -86,12 +93,12 @@ inline FwdPlan fwd_plan(bool f16, int B, int S_q, int S_kv, int D_qk, int D_v, b
         f.bytes = f.o_bytes + rows * 8;
     };
     if (!f16) {
-        divide(fwd_f32_parts(B, S_q, S_kv, pad(D_qk), pad(D_v), D_v, causal));
+        divide(fwd_f32_parts(B, S_q, S_kv, D_qk, D_v, causal));
         if (f.parts == 1) f.o_bytes = f.bytes = 0;
         return f;
     }
     const long long tiles = (long long)B * ((S_q + kSmallRows - 1) / kSmallRows);
-    const long long slots = pad(D_qk) + pad(D_v) <= 160 ? 512 : 256;
+    const long long slots = pad_dim(D_qk) + pad_dim(D_v) <= 160 ? 512 : 256;
     f.small = tiles <= (causal && S_q >= 1000 ? 2 * slots : slots);
     if (!f.small || causal || tiles > slots / 2) return f;
     const long long blocks = ((long long)S_kv + kSmallRows - 1) / kSmallRows;
@@ -155,6 +162,41 @@ inline bool dkdv_small(const AttnShape& s, bool causal) {
 // causal).  B 16, S_q 64, S_kv 4000: 115 -> 56.
 inline bool dq_ds_small(const AttnShape& s, bool causal) {
     return small_tiles(s.B, s.S_q, 64) <= (causal && s.S_q >= 1000 ? 1024 : 512);
+}
+
+// Workgroups that share a tile in the backward of a shape without a dS path
+// (D <= 64), and the floats of workspace their sums take: dQ tiles divided
+// over keys, fp32 also dK/dV tiles over queries.
+struct BwdParts {
+    int q, kv;
+    size_t dq_floats, dk_floats, dv_floats;
+    size_t floats() const { return dq_floats + dk_floats + dv_floats; }
+};
+
+inline BwdParts bwd_parts(bool f16, const AttnShape& s, bool causal) {
+    BwdParts r{1, 1, 0, 0, 0};
+    if (s.D_qk > 64 || s.D_v > 64 || s.B <= 0 || s.S_q <= 0 || s.S_kv <= 0) return r;
+    if (f16) {
+        r.q = dq_parts(s, causal);
+    } else {
+        // Blocks of 64 keys (dQ, 3.25 us measured at D = 64) and of 32 queries
+        // (dK/dV, 1.9).  Undivided -> chosen, us of the whole backward: B 8,
+        // S_q 64, S_kv 8000, D 64: 453 -> 94 (8 parts of dQ; more now); B 8,
+        // S 700, causal, D 64: 110 -> 80 (4 of dK/dV alone); B 20, S 400, D
+        // 32/4: 49.4 -> 41.5 (2 of dK/dV); B 64, S 512, causal: 100, undivided
+        // (in two parts of dQ 113).
+        const double cols = pad_dim(s.D_qk) + pad_dim(s.D_v);
+        r.q = least_time_parts((long long)s.B * ((s.S_q + 127) / 128), ((long long)s.S_kv + 63) / 64, causal,
+                               1.0 + 0.0175 * cols, 3, 8.0 * s.B * s.S_q * s.D_qk);
+        r.kv = least_time_parts((long long)s.B * ((s.S_kv + 127) / 128), ((long long)s.S_q + 31) / 32, causal,
+                                0.8 + 0.0085 * cols, 3, 8.0 * s.B * s.S_kv * (s.D_qk + s.D_v));
+    }
+    if (r.q > 1) r.dq_floats = (size_t)r.q * s.B * s.S_q * s.D_qk;
+    if (r.kv > 1) {
+        r.dk_floats = (size_t)r.kv * s.B * s.S_kv * s.D_qk;
+        r.dv_floats = (size_t)r.kv * s.B * s.S_kv * s.D_v;
+    }
+    return r;
 }
 
 }  // namespace sdpa
