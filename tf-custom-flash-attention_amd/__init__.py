@@ -134,9 +134,10 @@ def _dims(shape):
 
 def _u64(x) -> int:
     """Scalar seed/offset as uint64 (the reference reads scalar<uint64>)."""
-    import torch
-    if isinstance(x, torch.Tensor):
-        x = int(x.item())
+    if type(x) is not int:
+        import torch
+        if isinstance(x, torch.Tensor):
+            x = int(x.item())
     return int(x) & 0xFFFFFFFFFFFFFFFF
 
 
@@ -151,6 +152,10 @@ def _dtype_code(t) -> int:
 
 def _stream_handle(device) -> int:
     import torch
+    # the handle of torch.cuda.current_stream(device) without the Stream object
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None and device.index is not None:
+        return raw(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
@@ -177,6 +182,18 @@ def check_bwd(q, k, v, o, stats, d_o, seed=0, offset=0, causal_mask=False) -> No
                                             int(bool(causal_mask))))
 
 
+def _plain_fwd(torch, q, k, v, seed, offset, causal_mask) -> bool:
+    """Whether the arguments pass every check of ``check_fwd`` by a few
+    comparisons; anything else goes through it (building its ctypes arrays
+    took a third of a small call's host time)."""
+    if not (isinstance(q, torch.Tensor) and isinstance(k, torch.Tensor) and isinstance(v, torch.Tensor)
+            and type(seed) is int and type(offset) is int):
+        return False
+    sq, sk, sv = q.shape, k.shape, v.shape
+    return (len(sq) == len(sk) == len(sv) == 3 and sk[0] == sq[0] and sk[2] == sq[2] and sv[0] == sq[0]
+            and sv[1] == sk[1] and sq[2] <= 128 and sv[2] <= 128 and (not causal_mask or sq[1] == sk[1]))
+
+
 def sdpa(q, k, v, seed=0, offset=0, dropout: float = 0.0, scale: float = 1.0,
          causal_mask: bool = False):
     """Forward op ``Sdpa`` (sdpa_ops.cc:7-32): returns ``(o, stats)``.
@@ -185,7 +202,8 @@ def sdpa(q, k, v, seed=0, offset=0, dropout: float = 0.0, scale: float = 1.0,
     o [B,S_q,D_v] in that dtype, stats [B,S_q] fp32.
     """
     import torch
-    check_fwd(q, k, v, seed, offset, causal_mask)
+    if not _plain_fwd(torch, q, k, v, seed, offset, causal_mask):
+        check_fwd(q, k, v, seed, offset, causal_mask)
     if not (q.dtype == k.dtype == v.dtype):
         raise InvalidArgumentError("q, k and v must have the same dtype T")
     dt = _dtype_code(q)
@@ -215,7 +233,11 @@ def sdpa_grad(q, k, v, o, stats, d_o, seed=0, offset=0, dropout: float = 0.0,
     size over 64 then stores dS in the dK/dV kernel and forms dQ from it); False gives
     it the per-row workspace only, and both kernels form dS."""
     import torch
-    check_bwd(q, k, v, o, stats, d_o, seed, offset, causal_mask)
+    if not (_plain_fwd(torch, q, k, v, seed, offset, causal_mask) and isinstance(o, torch.Tensor)
+            and isinstance(stats, torch.Tensor) and isinstance(d_o, torch.Tensor)
+            and o.shape == (q.shape[0], q.shape[1], v.shape[2]) and d_o.shape == o.shape
+            and stats.shape == q.shape[:2]):
+        check_bwd(q, k, v, o, stats, d_o, seed, offset, causal_mask)
     if not (q.dtype == k.dtype == v.dtype == o.dtype == d_o.dtype):
         raise InvalidArgumentError("q, k, v, out and do must have the same dtype T")
     if stats.dtype != torch.float32:
