@@ -18,6 +18,8 @@ FWD = [
     (1, 31, 1551, 128, 64, False, 0.2, 6),   # parts of unequal length, a ragged tail
     (2, 32, 4096, 32, 128, False, 0.0, 16),  # two blocks per wave
     (5, 2, 3001, 64, 64, False, 1.5, 12),    # every element dropped
+    (2, 70, 100, 36, 4, False, 0.1, 1),      # features a multiple of 4 only, on either side
+    (2, 33, 2050, 20, 60, False, 0.0, 8),    # the same in parts
 ]
 
 
@@ -87,6 +89,23 @@ def test_f32_forward(pkg, O, case):
         assert maxabs(_np(o), o_ref) <= TOL["f32"]["o"] and maxabs(_np(s), s_ref) <= TOL["f32"]["stats"]
 
 
+def test_half4_neighbour_row(pkg):
+    """An infinity in a row does not reach the row before it, whose last chunk
+    is copied with the first features of that one."""
+    g = torch.Generator().manual_seed(2)
+    q, k, v = ((torch.rand((1, 64, 12), generator=g) + 0.1).half().cuda() for _ in range(3))
+    k[0, 7, 0] = float("-inf")  # key 7 weighs 0; key 6 keeps its weight
+    o, s = pkg.sdpa(q, k, v, scale=0.3)
+    ref = torch.softmax(q.double().cpu() @ k.double().cpu().transpose(1, 2) * 0.3, -1) @ v.double().cpu()
+    assert (o.double().cpu() - ref).abs().max().item() <= 2e-3
+    k[0, 7, 0] = 0.5
+    v[0, 9, 0] = float("inf")  # dP of key 8 stays finite
+    d_o = torch.randn((1, 64, 12), generator=g).half().cuda()
+    o = torch.zeros_like(q)
+    _, dk, _ = pkg.sdpa_grad(q, k, v, o, s, d_o, scale=0.3)
+    assert torch.isfinite(dk[0, 8].float()).all() and not torch.isfinite(dk[0, 9].float()).all()
+
+
 def test_f32_forward_extreme_keys(pkg):
     """A key of -inf scores weighs 0 (its bf16 parts are NaN past the first),
     and one near the type's lowest value as well; other rows keep their error."""
@@ -111,6 +130,8 @@ BWD = [
     ("f16", 2, 160, 160, 128, 128, True, 0.2, 1),   # dS path: sub-tiles that are not stored
     ("f16", 1, 98, 225, 128, 32, False, 0.1, 1),    # dS path, ragged on both sides
     ("f16", 1, 129, 70, 24, 72, False, 1.5, 1),     # dS path, every element dropped
+    ("f16", 2, 130, 130, 36, 4, True, 0.1, 1),      # features a multiple of 4 only
+    ("f16", 2, 35, 1100, 12, 60, False, 0.2, 4),    # the same, dQ in parts
     ("f32", 2, 33, 129, 64, 64, False, 0.1, 3),     # a one-row query block, a one-key tile
     ("f32", 1, 65, 65, 37, 5, True, 0.1, 1),        # element loads, the diagonal
     ("f32", 1, 33, 1100, 64, 64, False, 0.2, 2),    # dQ in parts, ragged

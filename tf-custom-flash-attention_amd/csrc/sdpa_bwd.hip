@@ -32,6 +32,7 @@
 #include "sdpa_device.h"
 #include "sdpa_launch.h"
 #include "sdpa_params.h"
+#include "sdpa_parts.h"
 #include "sdpa_tile.h"
 
 namespace sdpa {
@@ -663,7 +664,7 @@ void sdpa_bwd_dq_f32_kernel(const BwdParams p) {
 // ---------------------------------------------------------------------------
 // Host launcher: dQ (+ delta) first, then dK/dV, on the caller's stream.
 // ---------------------------------------------------------------------------
-hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, int phases, hipStream_t stream) {
+hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, bool half4, int phases, hipStream_t stream) {
     const int B = p.s.B, S_q = p.s.S_q, S_kv = p.s.S_kv;
     if (B == 0) return hipSuccess;
     const bool drop = p.c.use_dropout != 0;
@@ -679,9 +680,14 @@ hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, int phases, hip
                         using CK = BwdKVF16Cfg<DQK, DV>;
                         const unsigned gq = (unsigned)(((S_q + CQ::BM - 1) / CQ::BM) * B);
                         const unsigned gk = (unsigned)(((S_kv + CK::BKV - 1) / CK::BKV) * B);
-                        if (phases & kBwdDq)
+                        const bool causal = p.c.causal != 0;
+                        if ((phases & kBwdDq) && half4 && dq_small(p.s, causal))
+                            err = launch_bwd_dq_f16_wave(p, stream);
+                        else if (phases & kBwdDq)
                             err = launch_kernel<sdpa_bwd_dq_f16_kernel<DQK, DV, V, D>>(gq, CQ::NT, CQ::LDS_BYTES, stream, p);
-                        if (err == hipSuccess && (phases & kBwdDkDv))
+                        if (err == hipSuccess && (phases & kBwdDkDv) && half4 && dkdv_small(p.s, causal))
+                            err = launch_bwd_dkdv_f16_wave(p, stream);
+                        else if (err == hipSuccess && (phases & kBwdDkDv))
                             err = launch_kernel<sdpa_bwd_dkdv_f16_kernel<DQK, DV, V, D>>(gk, CK::NT, CK::LDS_BYTES, stream, p);
                     } else {
                         if (phases & kBwdDq) {

@@ -87,6 +87,16 @@ bool vec_ok(int dtype, int D_qk, int D_v, std::initializer_list<const void*> ptr
     return true;
 }
 
+// fp16 rows of a multiple of 4 features (up to 64), 8-byte aligned: what the
+// kernels for small grids take besides vec_ok (sdpa_wave.h, keep4).
+bool half4_ok(int dtype, int D_qk, int D_v, std::initializer_list<const void*> ptrs) {
+    if (dtype != SDPA_DTYPE_F16 || D_qk <= 0 || D_v <= 0 || D_qk % 4 != 0 || D_v % 4 != 0 || D_qk > 64 || D_v > 64) return false;
+    if (D_qk % 8 == 0 && D_v % 8 == 0) return false;  // 16-byte aligned rows: vec_ok's
+    for (const void* p : ptrs)
+        if (((uintptr_t)p & 7u) != 0) return false;
+    return true;
+}
+
 // keep[b, i, j] from the same hash code the attention kernels use.
 // use_dropout: 0 keeps every element, 1 applies the hash test, 2 drops every
 // element (dropout > 1).
@@ -162,6 +172,7 @@ int sdpa_hip_fwd_ws(int dtype, const void* q, const void* k, const void* v, void
     }
     if (dtype == SDPA_DTYPE_F16 && vec)
         return hip_status(plan.small ? sdpa::launch_fwd_f16_wave(p, stream) : sdpa::launch_fwd_f16_dma(p, stream));
+    if (plan.small && half4_ok(dtype, D_qk, D_v, {q, k, v, o})) return hip_status(sdpa::launch_fwd_f16_wave(p, stream));
     if (dtype == SDPA_DTYPE_F32) return hip_status(sdpa::launch_fwd_f32(p, vec, stream));
     return hip_status(sdpa::launch_fwd_f16(p, vec, stream));
 }
@@ -277,9 +288,12 @@ int bwd_entry(Mode mode, int phases, int dtype, const void* q, const void* k, co
             e = f16 ? sdpa::launch_bwd_dq_ds_f16(p, stream) : sdpa::launch_bwd_dq_ds_f32(p, stream);
         return hip_status(e);
     }
+    const bool half4 = half4_ok(dtype, D_qk, D_v,
+                                {q, k, v, d_o, want_rows ? o : nullptr, want_dq ? dq : nullptr,
+                                 want_kv ? dk : nullptr, want_kv ? dv : nullptr});
     // the parts' sums behind the row values
     const sdpa::BwdParts parts = sdpa::bwd_parts(dtype == SDPA_DTYPE_F16, p.s, causal_mask != 0);
-    if (mode == kAuto && (vec || dtype == SDPA_DTYPE_F32) && parts.floats() > 0 && aligned16(workspace) &&
+    if (mode == kAuto && (vec || half4 || dtype == SDPA_DTYPE_F32) && parts.floats() > 0 && aligned16(workspace) &&
         workspace_bytes >= rows_bytes + parts.floats() * sizeof(float)) {
         p.parts = parts.q;
         p.kv_parts = parts.kv;
@@ -289,7 +303,7 @@ int bwd_entry(Mode mode, int phases, int dtype, const void* q, const void* k, co
     }
     const int ph = mode == kAuto ? (sdpa::kBwdDq | sdpa::kBwdDkDv) : phases;
     if (dtype == SDPA_DTYPE_F16 && vec) return hip_status(sdpa::launch_bwd_f16_dma(p, ph, stream));
-    return hip_status(sdpa::launch_bwd(p, (sdpa::DType)dtype, vec, ph, stream));
+    return hip_status(sdpa::launch_bwd(p, (sdpa::DType)dtype, vec, half4, ph, stream));
 }
 }  // namespace
 

@@ -12,6 +12,10 @@
 // dQ kernel may further divide a tile's keys over workgroups, whose sums a
 // second kernel adds in part order from the caller's workspace.
 //
+// D <= 64 may also be a multiple of 4 only (P4, keep4), which the large
+// kernels' copies do not take: the register-staged kernels served such shapes
+// (step of B 20, S 400, D 32/4, dropout: 87 -> 32 us).
+//
 // Element semantics are those of the large kernels (sdpa_bwd.hip restates the
 // reference's, sdpa/sdpa_bwd.cu.cc:130-170, 291-327).
 #include <type_traits>
@@ -38,7 +42,7 @@ struct DqWaveCfg {
     static constexpr int COPIES = WaveCopy<LK, false>::LOADS + WaveCopy<LV, false>::LOADS;
 };
 
-template <int DQK, int DV, bool CAUSAL, bool DROP>
+template <int DQK, int DV, bool CAUSAL, bool DROP, bool P4>
 __global__ __launch_bounds__((DqWaveCfg<DQK, DV>::NT)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void sdpa_bwd_dq_f16_wave_kernel(const BwdParams p, const int win) {
     using Cfg = DqWaveCfg<DQK, DV>;
@@ -66,8 +70,8 @@ void sdpa_bwd_dq_f16_wave_kernel(const BwdParams p, const int win) {
     const uint32_t ringo = (uint32_t)(wave * Cfg::RING), ring = lds_base() + ringo;
     WaveCopy<LK, false> kc;
     WaveCopy<LV, false> vc;
-    kc.init(lane, D_qk * 2, D_qk / 8);
-    vc.init(lane, D_v * 2, D_v / 8);
+    kc.init(lane, D_qk * 2, (D_qk + 7) / 8);
+    vc.init(lane, D_v * 2, (D_v + 7) / 8);
     auto issue = [&](int blk, uint32_t so) {
         kc.issue(ksrc.shifted(blk * BN), ring + so);
         vc.issue(vsrc.shifted(blk * BN), ring + so + (uint32_t)Cfg::KB);
@@ -77,12 +81,12 @@ void sdpa_bwd_dq_f16_wave_kernel(const BwdParams p, const int win) {
     half8 qreg[NK], doreg[NV];
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks)
-        qreg[ks] = __builtin_bit_cast(half8, load_row_chunk<half_t, true>(Qb, my_q, S_q, 16 * ks + 8 * hh, D_qk, D_qk));
+        qreg[ks] = __builtin_bit_cast(half8, load_row_chunk<half_t, !P4>(Qb, my_q, S_q, 16 * ks + 8 * hh, D_qk, D_qk));
     float dpart = 0.f;
 #pragma unroll
     for (int ks = 0; ks < NV; ++ks) {
-        doreg[ks] = __builtin_bit_cast(half8, load_row_chunk<half_t, true>(dOb, my_q, S_q, 16 * ks + 8 * hh, D_v, D_v));
-        const half8 o8 = __builtin_bit_cast(half8, load_row_chunk<half_t, true>(Ob, my_q, S_q, 16 * ks + 8 * hh, D_v, D_v));
+        doreg[ks] = __builtin_bit_cast(half8, load_row_chunk<half_t, !P4>(dOb, my_q, S_q, 16 * ks + 8 * hh, D_v, D_v));
+        const half8 o8 = __builtin_bit_cast(half8, load_row_chunk<half_t, !P4>(Ob, my_q, S_q, 16 * ks + 8 * hh, D_v, D_v));
 #pragma unroll
         for (int e = 0; e < 8; ++e) dpart += (float)doreg[ks][e] * (float)o8[e];
     }
@@ -123,9 +127,9 @@ void sdpa_bwd_dq_f16_wave_kernel(const BwdParams p, const int win) {
         const uint32_t kb = ringo + so, vb = kb + (uint32_t)Cfg::KB;
         floatx16 s = floatx16{}, dp = floatx16{};
 #pragma unroll
-        for (int ks = 0; ks < NK; ++ks) s = mfma_f16(lds_row<LK>(kb + swK.row, ks, 0), qreg[ks], s);
+        for (int ks = 0; ks < NK; ++ks) s = mfma_f16(keep4<P4>(lds_row<LK>(kb + swK.row, ks, 0), ks, hh, D_qk), qreg[ks], s);
 #pragma unroll
-        for (int ks = 0; ks < NV; ++ks) dp = mfma_f16(lds_row<LV>(vb + swV.row, ks, 0), doreg[ks], dp);
+        for (int ks = 0; ks < NV; ++ks) dp = mfma_f16(keep4<P4>(lds_row<LV>(vb + swV.row, ks, 0), ks, hh, D_v), doreg[ks], dp);
         half8 at[2][NDT];
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -211,7 +215,7 @@ struct DkvWaveCfg {
 // fp16's normal range (as in sdpa_f16_dkdv_split.hip).
 constexpr float kPScale = 64.f;
 
-template <int DQK, int DV, bool CAUSAL, bool DROP, bool DS>
+template <int DQK, int DV, bool CAUSAL, bool DROP, bool DS, bool P4>
 __global__ __launch_bounds__((DkvWaveCfg<DQK, DV>::NT))
 __attribute__((amdgpu_waves_per_eu(DkvWaveCfg<DQK, DV>::WPE, DkvWaveCfg<DQK, DV>::WPE)))
 void sdpa_bwd_dkdv_f16_wave_kernel(const BwdParams p, const int win) {
@@ -239,8 +243,8 @@ void sdpa_bwd_dkdv_f16_wave_kernel(const BwdParams p, const int win) {
     const uint32_t ringo = (uint32_t)(wave * Cfg::RING), ring = lds_base() + ringo;
     WaveCopy<LQ, false> qc;
     WaveCopy<LO, false> oc;
-    qc.init(lane, D_qk * 2, D_qk / 8);
-    oc.init(lane, D_v * 2, D_v / 8);
+    qc.init(lane, D_qk * 2, (D_qk + 7) / 8);
+    oc.init(lane, D_v * 2, (D_v + 7) / 8);
     auto issue = [&](int qb, uint32_t so) {
         const int q0 = qb * BQ;
         qc.issue(qsrc.shifted(q0), ring + so);
@@ -253,10 +257,10 @@ void sdpa_bwd_dkdv_f16_wave_kernel(const BwdParams p, const int win) {
     half8 kreg[NK], vreg[NV];
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks)
-        kreg[ks] = __builtin_bit_cast(half8, load_row_chunk<half_t, true>(Kb, my_k, S_kv, 16 * ks + 8 * hh, D_qk, D_qk));
+        kreg[ks] = __builtin_bit_cast(half8, load_row_chunk<half_t, !P4>(Kb, my_k, S_kv, 16 * ks + 8 * hh, D_qk, D_qk));
 #pragma unroll
     for (int ks = 0; ks < NV; ++ks)
-        vreg[ks] = __builtin_bit_cast(half8, load_row_chunk<half_t, true>(Vb, my_k, S_kv, 16 * ks + 8 * hh, D_v, D_v));
+        vreg[ks] = __builtin_bit_cast(half8, load_row_chunk<half_t, !P4>(Vb, my_k, S_kv, 16 * ks + 8 * hh, D_v, D_v));
     prologue_loads_landed();
     if (qb0 + wave < nqb) issue(qb0 + wave, 0);
     // With dropout dS' = dS (1 - p) = P (keep ? dP - delta' : -delta') with
@@ -301,9 +305,9 @@ void sdpa_bwd_dkdv_f16_wave_kernel(const BwdParams p, const int win) {
         const float* Fs = reinterpret_cast<const float*>(smem + obase + Cfg::OB);
         floatx16 s = floatx16{}, dp = floatx16{};
 #pragma unroll
-        for (int ks = 0; ks < NK; ++ks) s = mfma_f16(lds_row<LQ>(qbase + swQ.row, ks, 0), kreg[ks], s);
+        for (int ks = 0; ks < NK; ++ks) s = mfma_f16(keep4<P4>(lds_row<LQ>(qbase + swQ.row, ks, 0), ks, hh, D_qk), kreg[ks], s);
 #pragma unroll
-        for (int ks = 0; ks < NV; ++ks) dp = mfma_f16(lds_row<LO>(obase + swO.row, ks, 0), vreg[ks], dp);
+        for (int ks = 0; ks < NV; ++ks) dp = mfma_f16(keep4<P4>(lds_row<LO>(obase + swO.row, ks, 0), ks, hh, D_v), vreg[ks], dp);
         // rows past S_q (their zero stats2 would make P = 2^kGateShift) and,
         // causal, keys after the query
         const bool mask = q0 + BQ > S_q || (CAUSAL && q0 < k0 + BKV - 1);
@@ -418,7 +422,7 @@ void sdpa_bwd_dq_ds_f16_wave_kernel(const BwdParams p, const int win) {
     const RowSrc ksrc = row_src(p.k, (size_t)b * S_kv, S_kv, D_qk * 2);
     const uint32_t ringo = (uint32_t)(wave * Cfg::RING), ring = lds_base() + ringo;
     WaveCopy<LK, true> kc;
-    kc.init(lane, D_qk * 2, D_qk / 8);
+    kc.init(lane, D_qk * 2, (D_qk + 7) / 8);
     const int nblk = (min(S_kv, CAUSAL ? q0 + BM : S_kv) + BN - 1) / BN;
     // A sub-tile the dK/dV kernel did not store (its queries all before the
     // key group, or past S_q) is copied from an empty range: zeros.
@@ -507,9 +511,15 @@ hipError_t launch_bwd_dq_f16_wave(const BwdParams& p, hipStream_t stream) {
                     if constexpr (DQK <= 64 && DV <= 64) {
                         using Cfg = DqWaveCfg<DQK, DV>;
                         const long long n = (long long)((S_q + Cfg::BM - 1) / Cfg::BM) * p.parts * B;
-                        hipError_t err = launch_kernel<sdpa_bwd_dq_f16_wave_kernel<DQK, DV, decltype(c)::value, decltype(d)::value>>(
-                            (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p,
-                            row_window((size_t)p.s.S_kv * (DQK + DV) * 2));
+                        constexpr bool CA = decltype(c)::value, DR = decltype(d)::value;
+                        const int win = row_window((size_t)p.s.S_kv * (DQK + DV) * 2);
+                        hipError_t err;
+                        if (p.s.D_qk % 8 == 0 && p.s.D_v % 8 == 0)
+                            err = launch_kernel<sdpa_bwd_dq_f16_wave_kernel<DQK, DV, CA, DR, false>>(
+                                (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p, win);
+                        else
+                            err = launch_kernel<sdpa_bwd_dq_f16_wave_kernel<DQK, DV, CA, DR, true>>(
+                                (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p, win);
                         if (err == hipSuccess && p.parts > 1) {
                             const long long th = (long long)B * S_q * (p.s.D_qk / 4);
                             err = launch_kernel<sdpa_bwd_dq_merge_f16_kernel>((unsigned)((th + 255) / 256), 256, 0, stream, p);
@@ -538,10 +548,15 @@ hipError_t launch_bwd_dkdv_f16_wave(const BwdParams& p, hipStream_t stream) {
                     const int win = row_window((size_t)p.s.S_q * (DQK + DV) * 2);
                     if constexpr (DQK == 128 || DV == 128) {
                         if (p.ds)
-                            return launch_kernel<sdpa_bwd_dkdv_f16_wave_kernel<DQK, DV, CA, DR, true>>(
+                            return launch_kernel<sdpa_bwd_dkdv_f16_wave_kernel<DQK, DV, CA, DR, true, false>>(
                                 n, Cfg::NT, Cfg::LDS_BYTES, stream, p, win);
                     }
-                    return launch_kernel<sdpa_bwd_dkdv_f16_wave_kernel<DQK, DV, CA, DR, false>>(
+                    if constexpr (DQK <= 64 && DV <= 64) {
+                        if (p.s.D_qk % 8 != 0 || p.s.D_v % 8 != 0)
+                            return launch_kernel<sdpa_bwd_dkdv_f16_wave_kernel<DQK, DV, CA, DR, false, true>>(
+                                n, Cfg::NT, Cfg::LDS_BYTES, stream, p, win);
+                    }
+                    return launch_kernel<sdpa_bwd_dkdv_f16_wave_kernel<DQK, DV, CA, DR, false, false>>(
                         n, Cfg::NT, Cfg::LDS_BYTES, stream, p, win);
                 });
             });

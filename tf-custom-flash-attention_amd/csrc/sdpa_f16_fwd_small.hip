@@ -43,7 +43,7 @@ struct FwdWaveCfg {
     static_assert(COPIES < 64, "vmcnt is 6 bits");
 };
 
-template <int DQK, int DV, bool CAUSAL, bool DROP>
+template <int DQK, int DV, bool CAUSAL, bool DROP, bool P4>
 __global__ __launch_bounds__((FwdWaveCfg<DQK, DV>::NT))
 __attribute__((amdgpu_waves_per_eu(FwdWaveCfg<DQK, DV>::WPE, FwdWaveCfg<DQK, DV>::WPE)))
 void sdpa_fwd_f16_wave_kernel(const FwdParams p, const int win) {
@@ -75,8 +75,8 @@ void sdpa_fwd_f16_wave_kernel(const FwdParams p, const int win) {
     const uint32_t ring = lds_base() + (uint32_t)(wave * Cfg::RING);
     WaveCopy<LK, false> kc;
     WaveCopy<LV, true> vc;
-    kc.init(lane, D_qk * 2, D_qk / 8);
-    vc.init(lane, D_v * 2, D_v / 8);
+    kc.init(lane, D_qk * 2, (D_qk + 7) / 8);
+    vc.init(lane, D_v * 2, (D_v + 7) / 8);
     auto issue = [&](int blk, uint32_t so) {
         kc.issue(ksrc.shifted(blk * BN), ring + so);
         vc.issue(vsrc.shifted(blk * BN), ring + so + (uint32_t)Cfg::KB);
@@ -84,7 +84,7 @@ void sdpa_fwd_f16_wave_kernel(const FwdParams p, const int win) {
     half8 qreg[NKS];
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
-        half8 v = __builtin_bit_cast(half8, load_row_chunk<half_t, true>(Qb, my_q, S_q, 16 * ks + 8 * hh, D_qk, D_qk));
+        half8 v = __builtin_bit_cast(half8, load_row_chunk<half_t, !P4>(Qb, my_q, S_q, 16 * ks + 8 * hh, D_qk, D_qk));
         qreg[ks] = neg ? -v : v;
     }
     prologue_loads_landed();
@@ -120,7 +120,7 @@ void sdpa_fwd_f16_wave_kernel(const FwdParams p, const int win) {
         const float split_thr = m_run + fast_log2(xhalf_sum(l_run)) + kSplitLog2;
         floatx16 s = floatx16{};
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) s = mfma_f16(ld_b128((rkl ^ (uint32_t)(32 * ks)) + so), qreg[ks], s);
+        for (int ks = 0; ks < NKS; ++ks) s = mfma_f16(keep4<P4>(ld_b128((rkl ^ (uint32_t)(32 * ks)) + so), ks, hh, D_qk), qreg[ks], s);
         half8 av[2][NDT];
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -255,9 +255,15 @@ hipError_t launch_fwd_f16_wave(const FwdParams& p, hipStream_t stream) {
                     using Cfg = FwdWaveCfg<DQK, DV>;
                     static_assert(Cfg::BM == kSmallRows && Cfg::BN == kSmallRows && Cfg::NW == kSmallWaves, "planned by fwd_plan");
                     const long long n = (long long)((S_q + Cfg::BM - 1) / Cfg::BM) * p.parts * B;
-                    const hipError_t err = launch_kernel<sdpa_fwd_f16_wave_kernel<DQK, DV, decltype(c)::value, decltype(d)::value>>(
-                        (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p,
-                        row_window((size_t)p.s.S_kv * (DQK + DV) * 2));
+                    constexpr bool CA = decltype(c)::value, DR = decltype(d)::value;
+                    const int win = row_window((size_t)p.s.S_kv * (DQK + DV) * 2);
+                    hipError_t err = hipErrorInvalidValue;
+                    if (p.s.D_qk % 8 == 0 && p.s.D_v % 8 == 0)
+                        err = launch_kernel<sdpa_fwd_f16_wave_kernel<DQK, DV, CA, DR, false>>((unsigned)n, Cfg::NT, Cfg::LDS_BYTES,
+                                                                                          stream, p, win);
+                    else if constexpr (DQK <= 64 && DV <= 64)
+                        err = launch_kernel<sdpa_fwd_f16_wave_kernel<DQK, DV, CA, DR, true>>((unsigned)n, Cfg::NT, Cfg::LDS_BYTES,
+                                                                                         stream, p, win);
                     return err == hipSuccess && p.parts > 1 ? launch_fwd_merge<half_t>(p, stream) : err;
                 });
             });

@@ -56,7 +56,9 @@ hipError_t launch_fwd_f16(const FwdParams& p, bool vec, hipStream_t stream);
 hipError_t launch_fwd_f32(const FwdParams& p, bool vec, hipStream_t stream);
 // phases: kBwdDq (dQ kernel, writes delta) and/or kBwdDkDv (reads delta).
 constexpr int kBwdDq = 1, kBwdDkDv = 2;
-hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, int phases, hipStream_t stream);
+// half4: fp16 rows of a multiple of 4 features that the kernels for small
+// grids take.
+hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, bool half4, int phases, hipStream_t stream);
 
 // fp16 kernels fed by HBM -> LDS copies (sdpa_f16_fwd.hip, sdpa_f16_dq.hip,
 // sdpa_f16_dkdv.hip).  They require D_qk and D_v to be multiples of 8 and

@@ -76,6 +76,24 @@ __device__ __forceinline__ void sum_waves(const float* m, int tid, int nrows, in
     }
 }
 
+// Row operands of tiles whose feature size D is a multiple of 4 but not of 8
+// (P4): the last chunk of a row, copied whole, ends in four features of the
+// next row.  They only meet zeros of the other operand, but infinities there
+// must not, so a reduction over features clears them; outputs past D are not
+// stored.  keep4: which dwords 2 and 3 of chunk 2 ks + hh this lane keeps.
+template <bool P4>
+__device__ __forceinline__ half8 keep4(half8 x, int ks, int hh, int D) {
+    if constexpr (P4) {
+        typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+        u4 u = __builtin_bit_cast(u4, x);
+        const uint32_t k = 16 * ks + 8 * hh + 4 < D ? ~0u : 0u;
+        u[2] &= k;
+        u[3] &= k;
+        return __builtin_bit_cast(half8, u);
+    }
+    return x;
+}
+
 __device__ __forceinline__ half4 scaled_h4(const floatx4& s, float f) {
     half4 h;
 #pragma unroll
