@@ -20,6 +20,7 @@ FWD = [
     (5, 2, 3001, 64, 64, False, 1.5, 12),    # every element dropped
     (2, 70, 100, 36, 4, False, 0.1, 1),      # features a multiple of 4 only, on either side
     (2, 33, 2050, 20, 60, False, 0.0, 8),    # the same in parts
+    (3, 2881, 1999, 128, 96, False, 0.1, 3),  # the 128-query kernel in parts, ragged
 ]
 
 

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void sdpa_bwd_dq_merge_f16_kernel(const BwdPar
     const size_t n = (size_t)p.s.B * p.s.S_q * cpr, i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     const floatx4* src = reinterpret_cast<const floatx4*>(p.part_dq) + i;
-    constexpr int U = 8;  // loads in flight before the first is used
+    constexpr int U = 4;  // loads in flight before the first is used
     floatx4 s = floatx4{};
     for (int k0 = 0; k0 < np; k0 += U) {
         floatx4 x[U];

@@ -16,6 +16,8 @@
 // blocks of 64 keys through an LDS ring (three deep when it fits, else two),
 // one barrier per block: each block's copy is issued one or two steps before
 // it is read.
+// Without the causal mask the keys of a tile may be divided over workgroups
+// (DIV; sdpa_parts.h), whose results a second kernel merges.
 // Workgroup ids are remapped XCD-major (xcd_map); under causal masking the
 // heaviest query tiles of a batch row run first.
 //
@@ -33,7 +35,9 @@
 
 #include "sdpa_dma.h"
 #include "sdpa_launch.h"
+#include "sdpa_merge.h"
 #include "sdpa_params.h"
+#include "sdpa_parts.h"
 
 namespace sdpa {
 namespace {
@@ -63,7 +67,7 @@ struct FwdDmaCfg {
     static_assert(KB + VB <= 65536, "LDS immediates");
 };
 
-template <int DQK, int DV, bool CAUSAL, bool DROP>
+template <int DQK, int DV, bool CAUSAL, bool DROP, bool DIV>
 __global__ __launch_bounds__((FwdDmaCfg<DQK, DV>::NT))
 __attribute__((amdgpu_waves_per_eu(FwdDmaCfg<DQK, DV>::template wpe<DROP>(), FwdDmaCfg<DQK, DV>::template wpe<DROP>())))
 void sdpa_fwd_f16_dma_kernel(const FwdParams p, const int win) {
@@ -74,9 +78,10 @@ void sdpa_fwd_f16_dma_kernel(const FwdParams p, const int win) {
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int B = p.s.B, S_q = p.s.S_q, S_kv = p.s.S_kv, D_qk = p.s.D_qk, D_v = p.s.D_v;
-    const int tiles = (S_q + BM - 1) / BM;
-    int b, qt;
-    xcd_map(blockIdx.x, B * tiles, tiles, CAUSAL, win, b, qt);
+    const int np = DIV ? p.parts : 1, items = (S_q + BM - 1) / BM * np;
+    int b, it;
+    xcd_map(blockIdx.x, B * items, items, CAUSAL, win, b, it);
+    const int qt = DIV ? it / np : it, part = DIV ? it - qt * np : 0;
     const int q0 = qt * BM, qw0 = q0 + 32 * wave, my_q = qw0 + l32;
 
     const half_t* Qb = static_cast<const half_t*>(p.q) + (size_t)b * S_q * D_qk;
@@ -108,7 +113,10 @@ void sdpa_fwd_f16_dma_kernel(const FwdParams p, const int win) {
     const uint32_t lds0 = lds_base();
     const uint32_t m0w = lds0 + 1024u * (uint32_t)wave;
     const int kv_end = CAUSAL ? min(S_kv, q0 + BM) : S_kv;
-    const int nsteps = (kv_end + BN - 1) / BN;
+    // the steps [lo, nsteps) of this workgroup (DIV: of this part of the keys)
+    const int steps = (kv_end + BN - 1) / BN;
+    const int lo = DIV ? part_begin(steps, part, np) : 0;
+    const int nsteps = DIV ? part_begin(steps, part + 1, np) : steps;
     // copy of key block `step` into its ring slot (step % NSTAGE)
     auto issue = [&](int step) {
         const int kv0 = step * BN;
@@ -120,7 +128,7 @@ void sdpa_fwd_f16_dma_kernel(const FwdParams p, const int win) {
     const int cpb = TileCopy<BN, LK, NW>::count(wave) + TileCopy<BN, LV, NW, true>::count(wave);
 #pragma unroll
     for (int i = 0; i < NSTAGE - 1; ++i)
-        if (i < nsteps) issue(i);
+        if (lo + i < nsteps) issue(lo + i);
 
     // ---- lane read addresses (the stage base and row offsets are added per
     // step / as instruction immediates).  The swizzle only permutes 16-byte
@@ -138,7 +146,9 @@ void sdpa_fwd_f16_dma_kernel(const FwdParams p, const int win) {
 
     // Dropout hash of (my_q, key 4 hh); element (key kv0 + c) adds (kv0 + c) A.
     // st_blk walks the key blocks: + BN A per step.
-    uint64_t st_blk = DROP ? lcg_state(p.c.seed_offset, (uint64_t)b * S_q + my_q, (uint64_t)S_kv, 4 * hh) : 0;
+    uint64_t st_blk = DROP ? lcg_state(p.c.seed_offset, (uint64_t)b * S_q + my_q, (uint64_t)S_kv,
+                                       (uint64_t)lo * BN + 4 * hh)
+                           : 0;
     const uint32_t thr = p.c.drop_threshold;
 
     // Softmax of one 32-key sub-tile t (scores s, raw q.k; masked keys set to
@@ -352,13 +362,30 @@ void sdpa_fwd_f16_dma_kernel(const FwdParams p, const int win) {
     // the unmasked variant; the causal diagonal and the key tail come last.
     const int full_lim = CAUSAL ? min(qw0 - (BN - 1), S_kv - BN) : S_kv - BN;
     const int n_full = qw0 >= S_q ? 0 : min(nsteps, full_lim < 0 ? 0 : full_lim / BN + 1);
-    int step = 0;
+    int step = lo;
     for (; step < n_full; ++step) do_step.template operator()<false>(step);
     for (; step < nsteps; ++step) do_step.template operator()<true>(step);
 
     // ---- epilogue: stats = m + log(l + 1e-6), O = acc / l (0 if l <= 1e-6) ----
     const float l_tot = xhalf_sum(l_run);
-    if (my_q < S_q) {
+    if (DIV && np > 1) {  // this part's unnormalised O, m and l
+        if (my_q < S_q) {
+            const size_t at = (size_t)part * B * S_q + (size_t)b * S_q + my_q;
+            if (hh == 0) {
+                p.part_ml[2 * at] = m_run;
+                p.part_ml[2 * at + 1] = l_tot;
+            }
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int d0 = 32 * dt + 8 * g + 4 * hh;
+                    if (d0 < D_v)
+                        *reinterpret_cast<floatx4*>(p.part_o + at * D_v + d0) =
+                            (floatx4){oacc[dt][4 * g], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+                }
+        }
+    } else if (my_q < S_q) {
         const float m_nat = (l_tot > 0.f) ? m_run * kLn2 : kNegInf;
         if (hh == 0) p.stats[(size_t)b * S_q + my_q] = m_nat + logf(l_tot + kEps);
         const float inv = (l_tot > kEps) ? p.c.keep_scale / l_tot : 0.f;
@@ -379,10 +406,18 @@ hipError_t launch_fwd_f16_dma(const FwdParams& p, hipStream_t stream) {
                 return with_bool(p.c.use_dropout != 0, [&](auto d) {
                     constexpr int DQK = decltype(dqk)::value, DV = decltype(dv)::value;
                     using Cfg = FwdDmaCfg<DQK, DV>;
-                    const long long n = (long long)((S_q + Cfg::BM - 1) / Cfg::BM) * B;
-                    return launch_kernel<sdpa_fwd_f16_dma_kernel<DQK, DV, decltype(c)::value, decltype(d)::value>>(
-                        (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p,
-                        row_window((size_t)p.s.S_kv * (DQK + DV) * 2));
+                    constexpr bool CA = decltype(c)::value, DR = decltype(d)::value;
+                    const long long n = (long long)((S_q + Cfg::BM - 1) / Cfg::BM) * p.parts * B;
+                    const int win = row_window((size_t)p.s.S_kv * (DQK + DV) * 2);
+                    if constexpr (!CA) {
+                        if (p.parts > 1) {
+                            const hipError_t err = launch_kernel<sdpa_fwd_f16_dma_kernel<DQK, DV, CA, DR, true>>(
+                                (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p, win);
+                            return err == hipSuccess ? launch_fwd_merge<half_t>(p, stream) : err;
+                        }
+                    }
+                    return launch_kernel<sdpa_fwd_f16_dma_kernel<DQK, DV, CA, DR, false>>((unsigned)n, Cfg::NT, Cfg::LDS_BYTES,
+                                                                                       stream, p, win);
                 });
             });
         });

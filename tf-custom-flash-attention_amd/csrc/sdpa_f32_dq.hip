@@ -181,7 +181,7 @@ void sdpa_bwd_dq_f32_bf3_kernel(const BwdParams p, const int win) {
         store_rows_f32<DQK, VEC>(static_cast<float*>(p.dq) + row_q * D_qk, dq, p.c.scale, hh, D_qk);
 }
 
-// dst[i] = f sum_k src[k n + i] over np parts, in part order.
+// dst[i] = f sum_k src[k n + i] over np parts, in part order; V values a thread.
 struct SumJob {
     float* dst;
     const float* src;
@@ -189,31 +189,36 @@ struct SumJob {
     int np;
     float f;
 };
-__global__ __launch_bounds__(256) void sdpa_bwd_merge_f32_kernel(const SumJob a, const SumJob b, const SumJob c) {
-    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const SumJob* j = &a;
-    if (i >= a.n) {
-        i -= a.n;
-        j = &b;
-        if (i >= b.n) {
-            i -= b.n;
-            j = &c;
-            if (i >= c.n) return;
-        }
-    }
-    constexpr int U = 8;  // loads in flight before the first is used
-    const int np = j->np;
-    const size_t n = j->n;
-    float s = 0.f;
-    for (int k0 = 0; k0 < np; k0 += U) {
-        float x[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = j->src[(size_t)(k0 + u < np ? k0 + u : np - 1) * n + i];
+template <int V>
+__device__ __forceinline__ void sum_parts(const SumJob& j, size_t i) {
+    typedef float vec __attribute__((ext_vector_type(V)));
+    vec s = vec{};
+    constexpr int U = 4;  // loads in flight before the first is used
+    for (int k0 = 0; k0 < j.np; k0 += U) {
+        vec x[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (k0 + u < np) s += x[u];
+            x[u] = *reinterpret_cast<const vec*>(j.src + (size_t)(k0 + u < j.np ? k0 + u : j.np - 1) * j.n + i);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (k0 + u < j.np) s += x[u];
     }
-    j->dst[i] = s * j->f;
+    s *= j.f;
+    if (((uintptr_t)(j.dst + i) & (sizeof(vec) - 1)) == 0) {
+        *reinterpret_cast<vec*>(j.dst + i) = s;
+    } else {
+#pragma unroll
+        for (int e = 0; e < V; ++e) j.dst[i + e] = s[e];
+    }
+}
+template <int V>
+__global__ __launch_bounds__(256) void sdpa_bwd_merge_f32_kernel(const SumJob a, const SumJob b, const SumJob c) {
+    size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * V;
+    if (i < a.n) return sum_parts<V>(a, i);
+    i -= a.n;
+    if (i < b.n) return sum_parts<V>(b, i);
+    i -= b.n;
+    if (i < c.n) sum_parts<V>(c, i);
 }
 
 }  // namespace
@@ -248,7 +253,9 @@ hipError_t launch_bwd_merge_f32(const BwdParams& p, hipStream_t stream) {
     const SumJob v = p.kv_parts > 1 ? SumJob{static_cast<float*>(p.dv), p.part_dv, rk * p.s.D_v, p.kv_parts, p.c.keep_scale} : none;
     const size_t n = q.n + k.n + v.n;
     if (n == 0) return hipSuccess;
-    return launch_kernel<sdpa_bwd_merge_f32_kernel>((unsigned)((n + 255) / 256), 256, 0, stream, q, k, v);
+    if (p.s.D_qk % 4 == 0 && p.s.D_v % 4 == 0)
+        return launch_kernel<sdpa_bwd_merge_f32_kernel<4>>((unsigned)((n / 4 + 255) / 256), 256, 0, stream, q, k, v);
+    return launch_kernel<sdpa_bwd_merge_f32_kernel<1>>((unsigned)((n + 255) / 256), 256, 0, stream, q, k, v);
 }
 
 }  // namespace sdpa

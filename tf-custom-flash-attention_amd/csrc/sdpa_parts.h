@@ -29,15 +29,15 @@ struct FwdPlan {
 // read, at 2.5 TB/s).  Under the causal mask a tile has half of the blocks
 // on average, one of them all.
 inline int least_time_parts(long long tiles, long long blocks, bool causal, double block_us, double merge_us,
-                            double part_bytes) {
-    if (tiles > 256 || blocks < 2) return 1;
+                            double part_bytes, int slots = 256) {
+    if (tiles > slots || blocks < 2) return 1;
     int best = 1;
     double best_us = 0;
     for (int n = 1; n <= blocks && n <= 64; ++n) {
         const double chain = 4 + (double)((blocks + n - 1) / n) * block_us;
-        double us = (double)((tiles * n + 255) / 256) * chain;
+        double us = (double)((tiles * n + slots - 1) / slots) * chain;
         if (causal) {
-            const double work = (double)tiles * (4 * n + 0.5 * blocks * block_us) / 256 + chain / 2;
+            const double work = (double)tiles * (4 * n + 0.5 * blocks * block_us) / slots + chain / 2;
             us = work > chain ? work : chain;
         }
         if (n > 1) us += merge_us + n * part_bytes / 2.5e6;
@@ -100,9 +100,25 @@ inline FwdPlan fwd_plan(bool f16, int B, int S_q, int S_kv, int D_qk, int D_v, b
     const long long tiles = (long long)B * ((S_q + kSmallRows - 1) / kSmallRows);
     const long long slots = pad_dim(D_qk) + pad_dim(D_v) <= 160 ? 512 : 256;
     f.small = tiles <= (causal && S_q >= 1000 ? 2 * slots : slots);
-    if (!f.small || causal || tiles > slots / 2) return f;
     const long long blocks = ((long long)S_kv + kSmallRows - 1) / kSmallRows;
     const long long walk = (blocks + kSmallWaves - 1) / kSmallWaves;  // blocks per wave, undivided
+    // The 128-query kernel with its keys divided, 512 workgroups at a time:
+    // where the 32-query one does not run, or has no workgroup to spare for a
+    // division and a longer walk (a block there takes 0.65 us, 1.05 at a
+    // 128-wide side).  B 32, S_q 300, S_kv 2000, D 128: 43 -> 33 (3 parts);
+    // B 32, S_q 400, S_kv 8000, D 128: 145 -> 81 (4); B 64, S_q 300, S_kv
+    // 1500, D 80: 39.9, in two parts 39.3.
+    if (!causal && (!f.small || tiles > slots / 2)) {
+        const long long big = (long long)B * ((S_q + 127) / 128), steps = ((long long)S_kv + 63) / 64;
+        const int n = least_time_parts(big, steps, false, 1.25, 8, 8.0 * B * S_q * D_v, 512);
+        const double big_us = 12 + (double)((steps + n - 1) / n) * 1.25 + n * 8.0 * B * S_q * D_v / 2.5e6;
+        if (n > 1 && (!f.small || big_us < 4 + walk * (slots == 512 ? 0.65 : 1.05))) {
+            f.small = false;
+            divide(n);
+            return f;
+        }
+    }
+    if (!f.small || causal || tiles > slots / 2) return f;
     long long n = 256 / tiles;
     if (slots == 512 && (n < 1 || walk / n >= 12)) n = slots / tiles;
     if (n > walk / 2) n = walk / 2;
