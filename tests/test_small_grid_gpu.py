@@ -64,6 +64,8 @@ F32 = [
     (2, 65, 65, 37, 5, True, 0.2, -0.2),         # element loads, negated scale
     (2, 200, 200, 32, 128, True, 0.1, 0.0),      # scale 0
     (3, 1, 700, 128, 64, False, 1.5, 0.1),       # every element dropped
+    (1, 17, 8193, 40, 36, False, 0.1, 0.16),     # the sequential fp32 sums (more than 8192 keys)
+    (1, 33, 8225, 126, 6, False, 0.0, 0.09),     # the same with rows of no whole chunks
 ]
 
 
@@ -140,6 +142,8 @@ BWD = [
     ("f32", 1, 513, 513, 64, 64, True, 1.5, 2),     # both, the diagonal, every element dropped
     ("f32", 2, 160, 160, 128, 128, True, 0.2, 1),   # dS path
     ("f32", 1, 31, 257, 128, 32, False, 1.5, 1),    # dS path, every element dropped
+    ("f32", 1, 17, 8193, 40, 36, False, 0.1, 1),    # the sequential fp32 sums, undivided
+    ("f32", 1, 33, 8225, 128, 64, False, 0.0, 1),   # the same, dS path
 ]
 
 

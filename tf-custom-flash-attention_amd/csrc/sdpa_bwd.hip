@@ -691,7 +691,7 @@ hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, bool half4, int
                             err = launch_kernel<sdpa_bwd_dkdv_f16_kernel<DQK, DV, V, D>>(gk, CK::NT, CK::LDS_BYTES, stream, p);
                     } else {
                         if (phases & kBwdDq) {
-                            if constexpr (DQK == 128 || DV == 128) {
+                            if (DQK == 128 || DV == 128 || fp32_chain(p.s)) {
                                 using CQ = BwdQF32Cfg<DQK, DV>;
                                 const unsigned gq = (unsigned)(((S_q + CQ::BM - 1) / CQ::BM) * B);
                                 err = launch_kernel<sdpa_bwd_dq_f32_kernel<DQK, DV, V, D>>(gq, CQ::NT, CQ::LDS_BYTES, stream, p);

@@ -263,6 +263,7 @@ void sdpa_bwd_dkdv_f32_bf3_kernel(const BwdParams p, const int win) {
 hipError_t launch_bwd_dkdv_f32(const BwdParams& p, bool vec, hipStream_t stream) {
     const int B = p.s.B, S_kv = p.s.S_kv;
     if (B == 0 || S_kv == 0) return hipSuccess;
+    if (fp32_chain(p.s)) return launch_bwd_dkdv_f32_chain(p, vec, stream);
     return with_dim(p.s.D_qk, [&](auto dqk) {
         return with_dim(p.s.D_v, [&](auto dv) {
             return with_bool(vec, [&](auto v) {

@@ -97,4 +97,8 @@ hipError_t launch_bwd_dkdv_f32(const BwdParams& p, bool vec, hipStream_t stream)
 hipError_t launch_bwd_rows_f32(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dq_ds_f32(const BwdParams& p, hipStream_t stream);
 
+// The fp32 forward and dK/dV of the shapes of fp32_chain() (sdpa_f32_chain.hip).
+hipError_t launch_fwd_f32_chain(const FwdParams& p, bool vec, hipStream_t stream);
+hipError_t launch_bwd_dkdv_f32_chain(const BwdParams& p, bool vec, hipStream_t stream);
+
 }  // namespace sdpa

@@ -57,7 +57,15 @@ inline int pad_dim(int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }
 // + 64, 2.95 for 32 keys at 128 + 128.  Undivided -> chosen, us: B 8, S_q 1,
 // S_kv 8000, D 64: 288 -> 22.6 (32 parts); B 64, S_q 64, S_kv 2000, D 128:
 // 194 -> 65 (4); B 24, S 700, D 64: 38 (1; in two parts 57: a second round).
+// fp32 shapes that keep the sequential fp32 sums of sdpa_f32_chain.hip, where
+// the gate of the gradient lies among the weights of ordinary rows (figures
+// there: none of 40 calls differed up to 12000 keys, 11 of 38 at 16384; for
+// scores of unit variance the weights near the gate grow 16-fold from 8192 to
+// 16384 keys).  Up to 16 queries are generation, which takes no gradient.
+inline bool fp32_chain(const AttnShape& s) { return s.S_kv > 8192 && s.S_q > 16; }
+
 inline int fwd_f32_parts(int B, int S_q, int S_kv, int D_qk, int D_v, bool causal) {
+    if (fp32_chain(AttnShape{B, S_q, S_kv, D_qk, D_v})) return 1;
     const int pq = pad_dim(D_qk), pv = pad_dim(D_v);
     const bool wide = pq == 128 && pv == 128;
     return least_time_parts((long long)B * ((S_q + 127) / 128), ((long long)S_kv + (wide ? 31 : 63)) / (wide ? 32 : 64),
@@ -194,7 +202,7 @@ inline BwdParts bwd_parts(bool f16, const AttnShape& s, bool causal) {
     if (s.D_qk > 64 || s.D_v > 64 || s.B <= 0 || s.S_q <= 0 || s.S_kv <= 0) return r;
     if (f16) {
         r.q = dq_parts(s, causal);
-    } else {
+    } else if (!fp32_chain(s)) {
         // Blocks of 64 keys (dQ, 3.25 us measured at D = 64) and of 32 queries
         // (dK/dV, 1.9).  Undivided -> chosen, us of the whole backward: B 8,
         // S_q 64, S_kv 8000, D 64: 453 -> 94 (8 parts of dQ; more now); B 8,
