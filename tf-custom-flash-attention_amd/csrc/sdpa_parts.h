@@ -51,12 +51,6 @@ inline int least_time_parts(long long tiles, long long blocks, bool causal, doub
 
 inline int pad_dim(int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }
 
-// Parts of the keys of a 128-query tile in the fp32 forward (sdpa_f32_fwd.hip).
-// A block (64 keys, 32 where both sides are 128 wide) takes about 0.0215 us
-// per padded feature column of K and V: 2.35 measured at 64 + 64, 4.2 at 128
-// + 64, 2.95 for 32 keys at 128 + 128.  Undivided -> chosen, us: B 8, S_q 1,
-// S_kv 8000, D 64: 288 -> 22.6 (32 parts); B 64, S_q 64, S_kv 2000, D 128:
-// 194 -> 65 (4); B 24, S 700, D 64: 38 (1; in two parts 57: a second round).
 // fp32 shapes that keep the sequential fp32 sums of sdpa_f32_chain.hip, where
 // the gate of the gradient lies among the weights of ordinary rows (figures
 // there: none of 40 calls differed up to 12000 keys, 11 of 38 at 16384; for
@@ -64,6 +58,12 @@ inline int pad_dim(int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }
 // 16384 keys).  Up to 16 queries are generation, which takes no gradient.
 inline bool fp32_chain(const AttnShape& s) { return s.S_kv > 8192 && s.S_q > 16; }
 
+// Parts of the keys of a 128-query tile in the fp32 forward (sdpa_f32_fwd.hip).
+// A block (64 keys, 32 where both sides are 128 wide) takes about 0.0215 us
+// per padded feature column of K and V: 2.35 measured at 64 + 64, 4.2 at 128
+// + 64, 2.95 for 32 keys at 128 + 128.  Undivided -> chosen, us: B 8, S_q 1,
+// S_kv 8000, D 64: 288 -> 22.6 (32 parts); B 64, S_q 64, S_kv 2000, D 128:
+// 194 -> 65 (4); B 24, S 700, D 64: 38 (1; in two parts 57: a second round).
 inline int fwd_f32_parts(int B, int S_q, int S_kv, int D_qk, int D_v, bool causal) {
     if (fp32_chain(AttnShape{B, S_q, S_kv, D_qk, D_v})) return 1;
     const int pq = pad_dim(D_qk), pv = pad_dim(D_v);
