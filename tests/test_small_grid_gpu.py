@@ -109,6 +109,41 @@ def test_half4_neighbour_row(pkg):
     assert torch.isfinite(dk[0, 8].float()).all() and not torch.isfinite(dk[0, 9].float()).all()
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D_qk,D_v,S_kv", [(36, 60, 50), (64, 64, 50), (12, 60, 1100)])
+def test_small_backward_large_dp(pkg, D_qk, D_v, S_kv, causal):
+    """A factor dP / (1-p) - delta of 4e8 (dO 30000, v 200: all finite) beside
+    weights that are 0, of a gated key and of masked ones, leaves dQ finite
+    and within the rounding of dS and of the result to fp16 (2^-10 of the sum
+    of its terms' magnitudes; 2^-24 below fp16's normal range, for a dS and for
+    the result) and that of the fp32 sums dP and delta, 64 terms of 2^-24 each,
+    which cancel in a row of one visible key."""
+    if causal and S_kv != 50:
+        pytest.skip("one long side only")
+    g = torch.Generator().manual_seed(0)
+    S_q = 50 if causal else 40
+    q, k = torch.randn((1, S_q, D_qk), generator=g).half(), torch.randn((1, S_kv, D_qk), generator=g).half()
+    v, d_o = torch.randn((1, S_kv, D_v), generator=g).half(), torch.randn((1, S_q, D_v), generator=g).half()
+    q[:, :, 0] = 4
+    v *= 0.05  # the factors of the other keys leave dS below 65504
+    k[0, 7], v[0, 7] = 0, 200
+    k[0, 7, 0] = -60  # a weight of 0
+    d_o[0, 25] = 30000
+    c = [t.cuda() for t in (q, k, v)]
+    o, s = pkg.sdpa(*c, scale=0.2, causal_mask=causal)
+    dq, _, _ = pkg.sdpa_grad(*c, o, s, d_o.cuda(), scale=0.2, causal_mask=causal)
+    Q, K, V, G, O_, st = (t.double().cpu() for t in (q, k, v, d_o, o, s))
+    p = torch.exp(Q @ K.transpose(1, 2) * 0.2 - st[..., None])
+    if causal:
+        p = p.tril()
+    p = torch.where(p <= 1e-6, 0.0, p)
+    ds = p * (G @ V.transpose(1, 2) - (G * O_).sum(2, keepdim=True))
+    assert 50 < ds[0, 25].abs().max() < 60000 and p[0, 25, 7] == 0
+    sums = p * (G.abs() @ V.abs().transpose(1, 2) + (G * O_).abs().sum(2, keepdim=True)) * 2.0 ** -18
+    bound = ((ds.abs() * 2.0 ** -10 + sums + 2.0 ** -24) @ K.abs()) * 0.2 + 2.0 ** -24
+    assert ((dq.double().cpu() - ds @ K * 0.2).abs() <= bound).all()
+
+
 def test_f32_forward_extreme_keys(pkg):
     """A key of -inf scores weighs 0 (its bf16 parts are NaN past the first),
     and one near the type's lowest value as well; other rows keep their error."""

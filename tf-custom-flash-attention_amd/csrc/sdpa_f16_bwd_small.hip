@@ -28,6 +28,19 @@
 namespace sdpa {
 namespace {
 
+// P of a score x = s scale log2(e) - stats log2(e), 0 where P <= 1e-6.  P4
+// compares, as the register-staged kernels of these shapes do; the other
+// shapes have kGateShift in x, as their large kernels do (in bits of x that
+// lie below the rounding of P to fp16).  kGateScale enters here and not the
+// factor that P meets: dP / (1-p) - delta times 2^106 passes the fp32 range
+// at 4e6, and a weight of 0 would make NaN of it.
+template <bool P4>
+__device__ __forceinline__ float gated(float x) {
+    const float pr = fast_exp2(x);
+    if constexpr (P4) return pr > kEps ? pr : 0.f;
+    return pr * kGateScale;
+}
+
 // ---------------------------------------------------------------------------
 // dQ of 32 queries (D <= 64), with the row values for the dK/dV kernel
 // ---------------------------------------------------------------------------
@@ -92,15 +105,15 @@ void sdpa_bwd_dq_f16_wave_kernel(const BwdParams p, const int win) {
     }
     const float delta = xhalf_sum(dpart);
     const bool row_ok = my_q < S_q;
-    const float stats2g = row_ok ? __builtin_fmaf(p.stats[row_q], kLog2e, kGateShift) : INFINITY;
+    const float stats = row_ok ? p.stats[row_q] : INFINITY;
     if (row_ok && hh == 0 && wave == 0 && part == 0) {
         p.delta[row_q] = delta;
-        p.stats2[row_q] = stats2g;
+        p.stats2[row_q] = __builtin_fmaf(stats, kLog2e, kGateShift);
     }
     prologue_loads_landed();
     if (lo + wave < hi) issue(lo + wave, 0);
-    const float sl2 = p.c.scale_log2, nst = -stats2g;
-    const float kscg = p.c.keep_scale * kGateScale, deltag = delta * kGateScale;
+    const float sl2 = p.c.scale_log2, ksc = p.c.keep_scale;
+    const float nst = P4 ? -(stats * kLog2e) : -__builtin_fmaf(stats, kLog2e, kGateShift);
 
     uint64_t st = DROP ? lcg_state(p.c.seed_offset, row_q, (uint64_t)S_kv, (uint64_t)((lo + wave) * BN + 4 * hh)) : 0;
     const uint32_t thr = p.c.drop_threshold;
@@ -148,10 +161,11 @@ void sdpa_bwd_dq_f16_wave_kernel(const BwdParams p, const int win) {
                     const int key = k0 + 8 * (rr >> 2) + 4 * hh + (rr & 3);
                     if (key >= S_kv || (CAUSAL && key > my_q)) x = -INFINITY;
                 }
-                float t = __builtin_fmaf(dp[rr], kscg, -deltag);
+                const float pr = gated<P4>(x);
+                float t = __builtin_fmaf(dp[rr], ksc, -delta);
                 if constexpr (DROP)
-                    t = lcg_keep(st + (uint64_t)(8 * (rr >> 2) + (rr & 3)) * kLcgMul, thr) ? t : -deltag;
-                ds2[e] = fast_exp2(x) * t;  // P' (0 where P <= 1e-6) times the scaled factor
+                    t = lcg_keep(st + (uint64_t)(8 * (rr >> 2) + (rr & 3)) * kLcgMul, thr) ? t : -delta;
+                ds2[e] = pr * t;
             }
             w[r >> 1] = pack_h2(ds2[0], ds2[1]);
         }
