@@ -144,6 +144,27 @@ def test_small_backward_large_dp(pkg, D_qk, D_v, S_kv, causal):
     assert ((dq.double().cpu() - ds @ K * 0.2).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("D", [36, 64])
+def test_small_dk_of_small_gradients(pkg, D):
+    """dK at dropout 0.9 and dO of 1e-3, where most of dS lies near fp16's
+    smallest normal value: dS and the result each round to half of 2^-10 at
+    most, 2.8e-4 in root mean square, 4e-4 together; twice that."""
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn((4, 512, D), generator=g).half().cuda() for _ in range(3))
+    d_o = (torch.randn((4, 512, D), generator=g) * 1e-3).half().cuda()
+    kw = dict(dropout=0.9, scale=D ** -0.5)
+    keep = pkg.dropout_keep_mask(4, 512, 512, 0.9, 5, 9).double()
+    o, s = pkg.sdpa(q, k, v, 5, 9, **kw)
+    _, dk, _ = pkg.sdpa_grad(q, k, v, o, s, d_o, 5, 9, **kw)
+    Q, K, V, G, O_, st = (t.double() for t in (q, k, v, d_o, o, s))
+    p = torch.exp(torch.bmm(Q, K.transpose(1, 2).contiguous()) * D ** -0.5 - st[..., None])
+    p = torch.where(p <= 1e-6, 0.0, p)
+    dp = torch.bmm(G, V.transpose(1, 2).contiguous()) * keep / (1 - float(np.float32(0.9)))
+    ds = p * (dp - (G * O_).sum(2, keepdim=True))
+    ref = torch.bmm(ds.transpose(1, 2).contiguous(), Q) * D ** -0.5
+    assert ((dk.double() - ref).norm() / ref.norm()).item() <= 8e-4
+
+
 def test_f32_forward_extreme_keys(pkg):
     """A key of -inf scores weighs 0 (its bf16 parts are NaN past the first),
     and one near the type's lowest value as well; other rows keep their error."""

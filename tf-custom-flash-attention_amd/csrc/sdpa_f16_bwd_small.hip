@@ -217,7 +217,7 @@ template <int DQK, int DV>
 struct DkvWaveCfg {
     static constexpr int NW = kSmallWaves, NT = 64 * NW, BKV = kSmallRows, BQ = 32;
     static constexpr int LQ = DQK / 8, LO = DV / 8;
-    static constexpr int QB = BQ * DQK * 2, OB = BQ * DV * 2, FB = 2 * 256;  // stats2 and delta: 64 floats each, 32 used
+    static constexpr int QB = BQ * DQK * 2, OB = BQ * DV * 2, FB = 2 * 256;  // stats (P4) or stats2, and delta: 64 floats each, 32 used
     static constexpr int STAGE = QB + OB + FB, RING = 2 * STAGE;
     static constexpr int MERGE = NW * BKV * (acc_stride(DQK) + acc_stride(DV)) * 4;
     static constexpr size_t LDS_BYTES = NW * RING > MERGE ? NW * RING : MERGE;
@@ -249,7 +249,7 @@ void sdpa_bwd_dkdv_f16_wave_kernel(const BwdParams p, const int win) {
     const half_t* Vb = static_cast<const half_t*>(p.v) + (size_t)b * S_kv * D_v;
     const RowSrc qsrc = row_src(p.q, (size_t)b * S_q, S_q, D_qk * 2);
     const RowSrc osrc = row_src(p.d_o, (size_t)b * S_q, S_q, D_v * 2);
-    const float* st2b = p.stats2 + (size_t)b * S_q;
+    const float* stb = (P4 ? p.stats : p.stats2) + (size_t)b * S_q;
     const float* deltab = p.delta + (size_t)b * S_q;
 
     // query blocks [qb0, nqb); this wave's: qb0 + wave, + NW, ...
@@ -264,7 +264,7 @@ void sdpa_bwd_dkdv_f16_wave_kernel(const BwdParams p, const int win) {
         qc.issue(qsrc.shifted(q0), ring + so);
         oc.issue(osrc.shifted(q0), ring + so + (uint32_t)Cfg::QB);
         unsigned char* f = smem + ringo + so + Cfg::QB + Cfg::OB;
-        dma4(make_rsrc(st2b + q0, (long long)(S_q - q0) * 4), f, lane * 4);
+        dma4(make_rsrc(stb + q0, (long long)(S_q - q0) * 4), f, lane * 4);
         dma4(make_rsrc(deltab + q0, (long long)(S_q - q0) * 4), f + 256, lane * 4);
     };
 
@@ -277,17 +277,22 @@ void sdpa_bwd_dkdv_f16_wave_kernel(const BwdParams p, const int win) {
         vreg[ks] = __builtin_bit_cast(half8, load_row_chunk<half_t, !P4>(Vb, my_k, S_kv, 16 * ks + 8 * hh, D_v, D_v));
     prologue_loads_landed();
     if (qb0 + wave < nqb) issue(qb0 + wave, 0);
-    // With dropout dS' = dS (1 - p) = P (keep ? dP - delta' : -delta') with
+    // At a 128-wide side, where dS may be stored, as in the split-role kernel:
+    // with dropout dS' = dS (1 - p) = P (keep ? dP - delta' : -delta') with
     // delta' = delta (1 - p), and dK is stored with scale / (1 - p).
     // keep_scale 0 (dropout > 1, every element dropped): dP from zero V rows,
-    // delta' = delta, so dS' = -P delta.
+    // delta' = delta, so dS' = -P delta.  Else dS itself, which keeps more bits
+    // above fp16's smallest normal value: dropout 0.9 with dO ~ 1e-3, error of
+    // dK against 64 bits 2.2e-3 with dS', 3.6e-4 with dS.
+    constexpr bool SCALED = DQK == 128 || DV == 128;
+    static_assert(SCALED || !DS, "stored dS is dS'");
     const float ksc = p.c.keep_scale;
-    const bool drop_all = DROP && ksc == 0.f;
+    const bool drop_all = SCALED && DROP && ksc == 0.f;
     if (drop_all) {
 #pragma unroll
         for (int ks = 0; ks < NV; ++ks) vreg[ks] = half8{};
     }
-    const float rksc = DROP && !drop_all ? 1.f / ksc : 1.f;
+    const float rksc = SCALED && DROP && !drop_all ? 1.f / ksc : 1.f;
     const float sl2 = p.c.scale_log2;
     const uint64_t row_step = (uint64_t)S_kv * kLcgMul;
     uint64_t st = DROP ? lcg_state(p.c.seed_offset, (uint64_t)b * S_q + (uint64_t)((qb0 + wave) * BQ + 4 * hh),
@@ -334,18 +339,18 @@ void sdpa_bwd_dkdv_f16_wave_kernel(const BwdParams p, const int win) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int r = 4 * g + e;
-                float x = __builtin_fmaf(s[r], sl2, -st4[e]);
+                float x = __builtin_fmaf(s[r], sl2, P4 ? -(st4[e] * kLog2e) : -st4[e]);
                 if (mask) {
                     const int q = q0 + 8 * g + 4 * hh + e;
                     if (q >= S_q || (CAUSAL && my_k > q)) x = -INFINITY;
                 }
-                const float pr = fast_exp2(x) * kGateScale;  // 0 where P <= 1e-6
+                const float pr = gated<P4>(x);
                 float pk = pr * kPScale, t;
                 if constexpr (DROP) {
-                    const float de = de4[e] * rksc;
+                    const float de = SCALED ? de4[e] * rksc : de4[e];
                     const bool keep = lcg_keep(st + (uint64_t)(8 * g + e) * row_step, thr);
                     pk = keep ? pk : 0.f;
-                    t = keep ? dp[r] - de : -de;
+                    t = keep ? (SCALED ? dp[r] - de : __builtin_fmaf(dp[r], ksc, -de)) : -de;
                 } else {
                     t = dp[r] - de4[e];
                 }
@@ -391,7 +396,7 @@ void sdpa_bwd_dkdv_f16_wave_kernel(const BwdParams p, const int win) {
     acc_to_lds<DV>(mv, wave * BKV + l32, dvacc, hh);
     __syncthreads();
     const size_t krow0 = (size_t)b * S_kv + k0;
-    const float fk = DROP && !drop_all ? p.c.scale * ksc : p.c.scale, fv = ksc * (1.f / kPScale);
+    const float fk = SCALED && DROP && !drop_all ? p.c.scale * ksc : p.c.scale, fv = ksc * (1.f / kPScale);
     sum_waves<NW, BKV, DQK>(mk, tid, S_kv - k0, D_qk, [&](int row, int c, const floatx4& sum) {
         *reinterpret_cast<half4*>(static_cast<half_t*>(p.dk) + (krow0 + row) * D_qk + c) = scaled_h4(sum, fk);
     });
