@@ -92,6 +92,22 @@ def test_f32_forward(pkg, O, case):
         assert maxabs(_np(o), o_ref) <= TOL["f32"]["o"] and maxabs(_np(s), s_ref) <= TOL["f32"]["stats"]
 
 
+@pytest.mark.parametrize("S_q,S_kv", [(16, 64), (16, 4000), (300, 2000)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_stats_without_values(pkg, dtype, S_q, S_kv):
+    """D_v = 0: o is empty, stats are those of the scores (also where other
+    value sizes would take the kernel of 32-query tiles or divided keys)."""
+    g = torch.Generator().manual_seed(4)
+    B = 2 if S_q == 16 else 32
+    q, k = (torch.randn((B, n, 64), generator=g).to(dtype).cuda() for n in (S_q, S_kv))
+    junk = torch.full((B * S_q,), 777.0, device="cuda")
+    del junk  # stats take its place
+    o, s = pkg.sdpa(q, k, torch.empty((B, S_kv, 0), dtype=dtype, device="cuda"), scale=0.1)
+    ref = torch.logsumexp(torch.bmm(q.double(), k.double().transpose(1, 2).contiguous()) * 0.1, -1)
+    assert o.shape == (B, S_q, 0)
+    assert (s.double() - ref).abs().max().item() <= TOL["f32"]["stats"]
+
+
 def test_half4_neighbour_row(pkg):
     """An infinity in a row does not reach the row before it, whose last chunk
     is copied with the first features of that one."""

@@ -93,7 +93,9 @@ inline int fwd_f32_parts(int B, int S_q, int S_kv, int D_qk, int D_v, bool causa
 // B 128, S_q 1, S_kv 1000, D 128: 14.5 in one, 18.7 in two.
 inline FwdPlan fwd_plan(bool f16, int B, int S_q, int S_kv, int D_qk, int D_v, bool causal) {
     FwdPlan f{false, 1, 0, 0};
-    if (B <= 0 || S_q <= 0) return f;
+    // (without values there is only stats to write, which the small kernel and
+    // the merge kernel write with a row's first columns)
+    if (B <= 0 || S_q <= 0 || D_v == 0) return f;
     const auto divide = [&](long long n) {
         f.parts = (int)n;
         const size_t rows = (size_t)f.parts * B * S_q;
