@@ -198,6 +198,23 @@ def test_ds_workspace_bytes(pkg):
     assert L.sdpa_hip_bwd_workspace_bytes_ds(1, 2, 64, 0, 128, 128, 0) == L.sdpa_hip_bwd_workspace_bytes(2, 64)
 
 
+def test_no_workspace_where_nothing_is_divided(pkg):
+    """fp16 widths that the register-staged kernels serve (which divide
+    nothing) ask for no more than the per-row workspace; widths a multiple of
+    4 only divide where the kernel of 32-query tiles runs."""
+    L = pkg.library()
+    for D_qk, D_v in ((63, 63), (64, 30), (12, 68), (100, 100)):
+        for B, S_q, S_kv in ((4, 16, 8192), (32, 300, 2000)):
+            dims = (1, B, S_q, S_kv, D_qk, D_v, 0)
+            assert L.sdpa_hip_fwd_workspace_bytes(*dims) == 0
+            assert L.sdpa_hip_bwd_workspace_bytes_full(*dims) == L.sdpa_hip_bwd_workspace_bytes_ds(*dims)
+    assert L.sdpa_hip_fwd_workspace_bytes(1, 4, 16, 8192, 36, 36, 0) > 0
+    assert L.sdpa_hip_fwd_workspace_bytes(1, 60, 300, 2000, 36, 36, 0) == 0  # 600 tiles: not the 32-query kernel
+    assert L.sdpa_hip_fwd_workspace_bytes(1, 32, 300, 2000, 128, 128, 0) > 0
+    # fp32 divides at any width
+    assert L.sdpa_hip_fwd_workspace_bytes(0, 4, 16, 8192, 63, 63, 0) > 0
+
+
 def test_ds_phase_rejects_before_device_work(pkg):
     """sdpa_hip_bwd_ds_phase returns SDPA_ERR_DS_PATH where sdpa_hip_bwd would
     not take the dS path; the stand-in addresses (16-byte aligned, never

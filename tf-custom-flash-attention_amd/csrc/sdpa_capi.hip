@@ -87,11 +87,10 @@ bool vec_ok(int dtype, int D_qk, int D_v, std::initializer_list<const void*> ptr
     return true;
 }
 
-// fp16 rows of a multiple of 4 features (up to 64), 8-byte aligned: what the
-// kernels for small grids take besides vec_ok (sdpa_wave.h, keep4).
+// fp16 rows of half chunks, 8-byte aligned: what the kernels for small grids
+// take besides vec_ok.
 bool half4_ok(int dtype, int D_qk, int D_v, std::initializer_list<const void*> ptrs) {
-    if (dtype != SDPA_DTYPE_F16 || D_qk <= 0 || D_v <= 0 || D_qk % 4 != 0 || D_v % 4 != 0 || D_qk > 64 || D_v > 64) return false;
-    if (D_qk % 8 == 0 && D_v % 8 == 0) return false;  // 16-byte aligned rows: vec_ok's
+    if (dtype != SDPA_DTYPE_F16 || !sdpa::half4_dims(D_qk, D_v)) return false;
     for (const void* p : ptrs)
         if (((uintptr_t)p & 7u) != 0) return false;
     return true;

@@ -16,6 +16,13 @@ __host__ __device__ inline int part_begin(int n, int part, int np) { return (int
 // Tile height and waves of the kernels for small grids.
 constexpr int kSmallRows = 32, kSmallWaves = 4;
 
+// fp16 feature sizes (multiples of 4 up to 64) that the kernels for small
+// grids take and the copies of whole 16-byte chunks do not (sdpa_wave.h, keep4).
+inline bool half4_dims(int D_qk, int D_v) {
+    return D_qk > 0 && D_v > 0 && D_qk % 4 == 0 && D_v % 4 == 0 && D_qk <= 64 && D_v <= 64 &&
+           !(D_qk % 8 == 0 && D_v % 8 == 0);
+}
+
 struct FwdPlan {
     bool small;             // the kernel for small grids
     int parts;              // workgroups that share a tile's keys (merged by a second kernel)
@@ -96,7 +103,12 @@ inline FwdPlan fwd_plan(bool f16, int B, int S_q, int S_kv, int D_qk, int D_v, b
     // (without values there is only stats to write, which the small kernel and
     // the merge kernel write with a row's first columns)
     if (B <= 0 || S_q <= 0 || D_v == 0) return f;
+    // fp16 widths that the register-staged kernel serves, which divides
+    // nothing; with rows of half chunks only the 32-query kernel divides
+    const bool chunks = D_qk % 8 == 0 && D_v % 8 == 0;
+    if (f16 && !chunks && !half4_dims(D_qk, D_v)) return f;
     const auto divide = [&](long long n) {
+        if (f16 && !f.small && !chunks) return;
         f.parts = (int)n;
         const size_t rows = (size_t)f.parts * B * S_q;
         f.o_bytes = (rows * D_v * 4 + 255) & ~(size_t)255;
@@ -203,7 +215,8 @@ inline BwdParts bwd_parts(bool f16, const AttnShape& s, bool causal) {
     BwdParts r{1, 1, 0, 0, 0};
     if (s.D_qk > 64 || s.D_v > 64 || s.B <= 0 || s.S_q <= 0 || s.S_kv <= 0) return r;
     if (f16) {
-        r.q = dq_parts(s, causal);
+        // (the register-staged kernel of other widths divides nothing)
+        if ((s.D_qk % 8 == 0 && s.D_v % 8 == 0) || half4_dims(s.D_qk, s.D_v)) r.q = dq_parts(s, causal);
     } else if (!fp32_chain(s)) {
         // Blocks of 64 keys (dQ, 3.25 us measured at D = 64) and of 32 queries
         // (dK/dV, 1.9).  Undivided -> chosen, us of the whole backward: B 8,
