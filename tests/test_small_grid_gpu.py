@@ -108,6 +108,22 @@ def test_stats_without_values(pkg, dtype, S_q, S_kv):
     assert (s.double() - ref).abs().max().item() <= TOL["f32"]["stats"]
 
 
+def test_f32_grid_of_more_threads_than_one_dimension(pkg):
+    """2^23 + 5 batch rows of one query and one key: with 512 threads per tile
+    more than the 2^32 - 1 threads of a grid dimension.  The one weight is 1,
+    so o = v (times 1 / (1 + 1e-6), within the op's 1e-5), dV = dO and dQ = dK = 0,
+    each to the rounding of P and of sums of two terms below 40."""
+    B = (1 << 23) + 5
+    g = torch.Generator(device="cuda").manual_seed(6)
+    q, k, v, d_o = (torch.randn((B, 1, 2), generator=g, device="cuda") for _ in range(4))
+    o, s = pkg.sdpa(q, k, v, scale=0.5)
+    dq, dk, dv = pkg.sdpa_grad(q, k, v, o, s, d_o, scale=0.5)
+    assert (o - v).abs().max().item() <= 1e-5
+    assert (s - (q * k).sum(2) * 0.5).abs().max().item() <= 1e-4
+    assert (dv - d_o).abs().max().item() <= 1e-4
+    assert dq.abs().max().item() <= 1e-4 and dk.abs().max().item() <= 1e-4
+
+
 def test_half4_neighbour_row(pkg):
     """An infinity in a row does not reach the row before it, whose last chunk
     is copied with the first features of that one."""

@@ -54,7 +54,9 @@ void sdpa_bwd_dkdv_f32_bf3_kernel(const BwdParams p, const int win) {
     const bool causal = p.c.causal != 0;
     const int np = p.kv_parts, items = (S_kv + BKV - 1) / BKV * np;
     int b, it;
-    xcd_map(blockIdx.x, B * items, items, false, win, b, it);
+    const int id = tile_id();
+    if (id >= B * items) return;
+    xcd_map(id, B * items, items, false, win, b, it);
     const int kt = it / np, part = it - kt * np;
     const int k0 = kt * BKV, kw0 = k0 + kw * 32, my_k = kw0 + l32;
     const bool key_ok = my_k < S_kv, wave_live = kw0 < S_kv;
@@ -272,7 +274,7 @@ hipError_t launch_bwd_dkdv_f32(const BwdParams& p, bool vec, hipStream_t stream)
                     constexpr bool V = decltype(v)::value, D = decltype(d)::value;
                     using Cfg = DkvBf3Cfg<DQK, DV>;
                     static_assert(Cfg::BKV == DsLayout32::KT && Cfg::BQ == DsLayout32::QBK, "dS chunk geometry");
-                    const unsigned n = (unsigned)((long long)((S_kv + Cfg::BKV - 1) / Cfg::BKV) * p.kv_parts * B);
+                    const dim3 n = tile_grid((long long)((S_kv + Cfg::BKV - 1) / Cfg::BKV) * p.kv_parts * B, Cfg::NT);
                     const int win = row_window((size_t)p.s.S_q * (DQK + DV) * 4);
                     if constexpr (V && (DQK == 128 || DV == 128)) {
                         if (p.ds)

@@ -44,7 +44,9 @@ void sdpa_bwd_dq_f32_bf3_kernel(const BwdParams p, const int win) {
     const bool causal = p.c.causal != 0;
     const int np = p.parts, items = (S_q + BM - 1) / BM * np;
     int b, it;
-    xcd_map(blockIdx.x, B * items, items, causal, win, b, it);
+    const int id = tile_id();
+    if (id >= B * items) return;
+    xcd_map(id, B * items, items, causal, win, b, it);
     const int qt = it / np, part = it - qt * np;
     const int q0 = qt * BM, qw0 = q0 + wq * 32, my_q = qw0 + l32;
     const size_t row_q = (size_t)b * S_q + my_q;
@@ -233,9 +235,9 @@ hipError_t launch_bwd_dq_f32(const BwdParams& p, bool vec, hipStream_t stream) {
                     constexpr int DQK = decltype(dqk)::value, DV = decltype(dv)::value;
                     if constexpr (DQK <= 64 && DV <= 64) {
                         using Cfg = DqBf3Cfg<DQK, DV>;
-                        const unsigned n = (unsigned)((long long)((S_q + Cfg::BM - 1) / Cfg::BM) * p.parts * B);
+                        const long long n = (long long)((S_q + Cfg::BM - 1) / Cfg::BM) * p.parts * B;
                         return launch_kernel<sdpa_bwd_dq_f32_bf3_kernel<DQK, DV, decltype(v)::value, decltype(d)::value>>(
-                            n, Cfg::NT, Cfg::LDS_BYTES, stream, p, row_window((size_t)p.s.S_kv * (DQK + DV) * 4));
+                            tile_grid(n, Cfg::NT), Cfg::NT, Cfg::LDS_BYTES, stream, p, row_window((size_t)p.s.S_kv * (DQK + DV) * 4));
                     } else {
                         return hipErrorInvalidValue;
                     }

@@ -91,7 +91,9 @@ void sdpa_bwd_dq_ds_f32_kernel(const BwdParams p, const int win) {
     const int B = p.s.B, S_q = p.s.S_q, S_kv = p.s.S_kv, D_qk = p.s.D_qk;
     const int tiles = (S_q + BM - 1) / BM;
     int b, qt;
-    xcd_map(blockIdx.x, B * tiles, tiles, CAUSAL, win, b, qt);
+    const int id = tile_id();
+    if (id >= B * tiles) return;
+    xcd_map(id, B * tiles, tiles, CAUSAL, win, b, qt);
     const int qw0 = qt * BM + 32 * wq, qb = qw0 / DsLayout32::QBK;
     const int pq = 8 * ((l32 >> 2) & 3) + 4 * (l32 >> 4) + (l32 & 3);  // stored position -> query
     const DsLayout32 dsl(S_q, S_kv, CAUSAL);
@@ -198,7 +200,7 @@ hipError_t launch_bwd_dq_ds_f32(const BwdParams& p, hipStream_t stream) {
             using Cfg = DqDs32Cfg<DQK>;
             const long long n = (long long)((S_q + Cfg::BM - 1) / Cfg::BM) * B;
             return launch_kernel<sdpa_bwd_dq_ds_f32_kernel<DQK, decltype(c)::value>>(
-                (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p, row_window((size_t)p.s.S_kv * DQK * 4));
+                tile_grid(n, Cfg::NT), Cfg::NT, Cfg::LDS_BYTES, stream, p, row_window((size_t)p.s.S_kv * DQK * 4));
         });
     });
 }

@@ -58,7 +58,9 @@ void sdpa_fwd_f32_bf3_kernel(const FwdParams p, const int win) {
     const bool causal = p.c.causal != 0;
     const int np = p.parts, items = (S_q + BM - 1) / BM * np;
     int b, it;
-    xcd_map(blockIdx.x, B * items, items, causal, win, b, it);
+    const int id = tile_id();
+    if (id >= B * items) return;
+    xcd_map(id, B * items, items, causal, win, b, it);
     const int qt = it / np, part = it - qt * np;
     const int q0 = qt * BM, qw0 = q0 + wq * 32, my_q = qw0 + l32;
 
@@ -253,7 +255,7 @@ hipError_t launch_fwd_f32(const FwdParams& p, bool vec, hipStream_t stream) {
                     using Cfg = FwdBf3Cfg<DQK, DV>;
                     const long long n = (long long)((S_q + Cfg::BM - 1) / Cfg::BM) * p.parts * B;
                     const hipError_t err = launch_kernel<sdpa_fwd_f32_bf3_kernel<DQK, DV, decltype(v)::value, decltype(d)::value>>(
-                        (unsigned)n, Cfg::NT, Cfg::LDS_BYTES, stream, p, row_window((size_t)p.s.S_kv * (DQK + DV) * 4));
+                        tile_grid(n, Cfg::NT), Cfg::NT, Cfg::LDS_BYTES, stream, p, row_window((size_t)p.s.S_kv * (DQK + DV) * 4));
                     return err == hipSuccess && p.parts > 1 ? launch_fwd_merge<float>(p, stream) : err;
                 });
             });

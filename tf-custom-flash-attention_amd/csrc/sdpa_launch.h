@@ -31,12 +31,22 @@ hipError_t with_bool(bool b, F&& f) {
     return f(std::false_type{});
 }
 
+// Grid of n workgroups: one dimension, or rows of 2^22 where that would pass
+// the 2^32 - 1 threads HIP launches per dimension (tiles of 512 threads: 2^23
+// batch rows of up to 128 queries).  The kernel takes tile_id() and leaves
+// where it is n or more.
+inline dim3 tile_grid(long long n, unsigned block) {
+    if (n * block <= 0xFFFFFFFFll) return dim3((unsigned)n);
+    return dim3(1u << 22, (unsigned)((n + (1 << 22) - 1) >> 22));
+}
+__device__ __forceinline__ int tile_id() { return (int)(blockIdx.x + gridDim.x * blockIdx.y); }
+
 // Launch `kern` with `lds` bytes of dynamic LDS.  The per-kernel attribute is
-// set once per process (gfx950 has 160 KB of LDS per CU; kernels here use at
-// most ~100 KB).
+// set once per process (gfx950 has 160 KB of LDS per CU; kernels here use up
+// to all of it, which each checks).
 // The kernel is a template argument so that each kernel gets its own once-flag.
 template <auto kern, typename... Args>
-hipError_t launch_kernel(unsigned grid, unsigned block, size_t lds, hipStream_t stream,
+hipError_t launch_kernel(dim3 grid, unsigned block, size_t lds, hipStream_t stream,
                          const Args&... args) {
     static std::once_flag once;
     static hipError_t attr_err = hipSuccess;
@@ -45,8 +55,9 @@ hipError_t launch_kernel(unsigned grid, unsigned block, size_t lds, hipStream_t 
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
     if (attr_err != hipSuccess) return attr_err;
-    if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, stream, args...);
+    if (grid.x == 0) return hipSuccess;
+    if ((unsigned long long)grid.x * block > 0xFFFFFFFFull) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL(kern, grid, dim3(block), lds, stream, args...);
     return hipGetLastError();
 }
 
