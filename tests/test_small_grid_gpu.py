@@ -211,6 +211,93 @@ def test_f32_forward_extreme_keys(pkg):
     assert (o.double().cpu() - ref).abs().max().item() <= 1e-5
 
 
+# D_qk, D_v, S_kv: up to 8192 keys on the bf16 matrix cores (whole chunks and
+# element loads, both dQ paths, keys in parts), past that on the fp32 ones.
+INF = [(64, 64, 64), (37, 5, 128), (128, 64, 128), (128, 128, 128), (32, 128, 64), (64, 32, 2048), (64, 64, 8256)]
+
+
+def _same_class(got, ref, tol):
+    """Infinite and NaN where the reference is, the rest within tol."""
+    got, fin = got.double().cpu(), torch.isfinite(ref)
+    assert torch.equal(got[~fin].nan_to_num(nan=7.0), ref[~fin].nan_to_num(nan=7.0))
+    assert (got - ref)[fin].abs().max().item() <= tol * max(1.0, ref[fin].abs().max().item())
+
+
+@pytest.mark.parametrize("D_qk,D_v,S_kv", INF)
+def test_f32_forward_infinite_values(pkg, D_qk, D_v, S_kv):
+    """An infinite v makes o infinite in its feature (every weight is > 0), and
+    a NaN NaN; other features keep their error."""
+    g = torch.Generator().manual_seed(8)
+    q, k, v = (torch.randn((2, n, d), generator=g) for n, d in ((33, D_qk), (S_kv, D_qk), (S_kv, D_v)))
+    v[0, 5, 3] = v[0, 9, 3] = v[1, S_kv - 1, 0] = float("inf")
+    v[0, 6, 4] = float("-inf")
+    v[0, 7, 2] = float("nan")
+    o, s = pkg.sdpa(*(t.cuda() for t in (q, k, v)), scale=0.1)
+    x = q.double() @ k.double().transpose(1, 2) * 0.1
+    ref = torch.softmax(x, -1) @ v.double()
+    assert torch.isinf(ref[0, :, 3:5]).all() and torch.isnan(ref[0, :, 2]).all() and torch.isfinite(ref[0, :, :2]).all()
+    _same_class(o, ref, 1e-5)
+    assert (s.double().cpu() - torch.logsumexp(x, -1)).abs().max().item() <= TOL["f32"]["stats"]
+
+
+@pytest.mark.parametrize("what", ["d_o", "v"])
+@pytest.mark.parametrize("D_qk,D_v,S_kv", INF)
+def test_f32_backward_infinite_values(pkg, D_qk, D_v, S_kv, what):
+    """An infinite dO makes dV infinite in its feature, and dS of its row; an
+    infinite v makes dS of its key so; dQ and dK take the infinities whose
+    factors have one sign, and NaN of the others.  S_q and S_kv fill whole
+    tiles: a row of zeros beside an infinity is NaN in 32-row tiles."""
+    g = torch.Generator().manual_seed(9)
+    S_q = 64
+    q, k, v = (torch.randn((2, n, d), generator=g) for n, d in ((S_q, D_qk), (S_kv, D_qk), (S_kv, D_v)))
+    q *= 0.5  # every weight well over 1e-6
+    d_o = torch.randn((2, S_q, D_v), generator=g)
+    q[..., 0], k[..., 0] = q[..., 0].abs() + 0.1, k[..., 0].abs() + 0.1
+    o, s = pkg.sdpa(*(t.cuda() for t in (q, k, v)), scale=0.1)
+    o = o.cpu()
+    if what == "d_o":
+        v[0, :, 1] = v[0, :, 1].abs() + 0.1
+        d_o[0, 3, 1] = float("inf")
+        o[0, 3, 1] = -1.0  # delta -inf: dS of row 3 is +inf
+    else:
+        d_o[0, :, 3] = d_o[0, :, 3].abs() + 0.1
+        v[0, 5, 3] = float("inf")
+    got = pkg.sdpa_grad(*(t.cuda() for t in (q, k, v, o)), s, d_o.cuda(), scale=0.1)
+    Q, K, V, G, O_, st = (t.double() for t in (q, k, v, d_o, o, s.cpu()))
+    p = torch.exp(Q @ K.transpose(1, 2) * 0.1 - st[..., None])
+    assert (p > 2e-6).all()
+    ds = p * (G @ V.transpose(1, 2) - (G * O_).sum(2, keepdim=True))
+    ref = ds @ K * 0.1, ds.transpose(1, 2) @ Q * 0.1, p.transpose(1, 2) @ G
+    if what == "d_o":
+        assert torch.isinf(ref[2][0, :, 1]).all() and torch.isinf(ref[1][0]).all() and torch.isinf(ref[0][0, 3, 0])
+    else:
+        assert torch.isinf(ref[0][0]).all() and torch.isinf(ref[1][0, 5, 0]) and torch.isfinite(ref[2]).all()
+    for a, b in zip(got, ref):
+        _same_class(a, b, TOL["f32"]["grad"])
+
+
+@pytest.mark.parametrize("D", [64, 37, 128])
+def test_f32_backward_extreme_keys(pkg, D):
+    """A key of -inf scores weighs 0 in the gradient too: dK and dV of the
+    other keys keep their error, its own are 0, and dQ is NaN (0 times -inf)
+    in the one feature that holds the infinity."""
+    g = torch.Generator().manual_seed(10)
+    q, k, v, d_o = (torch.randn((2, 64, D), generator=g) for _ in range(4))
+    q[..., 3] = 1.0
+    k[0, 5, 3] = float("-inf")
+    o, s = pkg.sdpa(*(t.cuda() for t in (q, k, v)), scale=0.1)
+    dq, dk, dv = pkg.sdpa_grad(*(t.cuda() for t in (q, k, v)), o, s, d_o.cuda(), scale=0.1)
+    Q, K, V, G, O_, st = (t.double().cpu() for t in (q, k, v, d_o, o, s))
+    p = torch.exp(Q @ K.transpose(1, 2) * 0.1 - st[..., None])
+    assert (p[0, :, 5] == 0).all() and (p > 2e-6).sum() == p.numel() - 64
+    ds = p * (G @ V.transpose(1, 2) - (G * O_).sum(2, keepdim=True))
+    _same_class(dv, p.transpose(1, 2) @ G, TOL["f32"]["grad"])
+    _same_class(dk, ds.transpose(1, 2) @ Q * 0.1, TOL["f32"]["grad"])
+    ref = ds @ K.nan_to_num(neginf=0.0) * 0.1
+    ref[0, :, 3] = float("nan")
+    _same_class(dq, ref, TOL["f32"]["grad"])
+
+
 BWD = [
     # dtype, B, S_q, S_kv, D_qk, D_v, causal, dropout; parts of a tile in dQ and, fp32, in dK/dV
     ("f16", 2, 97, 65, 64, 64, False, 0.1, 1),      # every wave one query block, a one-key tile

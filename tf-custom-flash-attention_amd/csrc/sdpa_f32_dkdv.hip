@@ -85,24 +85,30 @@ void sdpa_bwd_dkdv_f32_bf3_kernel(const BwdParams p, const int win) {
             else fpre = r < S_q ? deltab[r] : 0.f;
         }
     };
-    auto store_block = [&](int qb) {
+    auto store_block = [&](int qb, auto inf) {
+        constexpr bool INF = decltype(inf)::value;
         unsigned char* st = smem + ((qb - qb0) & 1) * Cfg::STAGE;
         qst.store(st, tid);
-        ost.store(st + QT::BYTES, tid);
+        ost.template store<INF>(st + QT::BYTES, tid);
         if (tid < 2 * BQ) reinterpret_cast<float*>(st + QT::BYTES + OT::BYTES)[tid] = fpre;
     };
-    auto stage_next = [&](int qb) {
+    auto stage_next = [&](int qb, auto inf) {
         if (qb + 1 < nqb) {
-            store_block(qb + 1);
+            store_block(qb + 1, inf);
             if (qb + 2 < nqb) load_block(qb + 2);
         }
     };
     float* xs = reinterpret_cast<float*>(smem + 2 * Cfg::STAGE) + kw * 1024;  // this key group's P
-    if (qb0 < nqb) {
-        load_block(qb0);
-        store_block(qb0);
-        if (qb0 + 1 < nqb) load_block(qb0 + 1);
-    }
+    auto stage_first = [&](auto inf) {
+        if (qb0 < nqb) {
+            load_block(qb0);
+            store_block(qb0, inf);
+            if (qb0 + 1 < nqb) load_block(qb0 + 1);
+        }
+    };
+    // Each role passes over the blocks; INF: again, for infinities in dO, V or
+    // dS (sdpa_bf3.h), which either role may find
+    stage_first(std::false_type{});
     SwzLane<LQ> swQ;
     SwzLane<LO> swO;
     swQ.init(lane);
@@ -117,75 +123,82 @@ void sdpa_bwd_dkdv_f32_bf3_kernel(const BwdParams p, const int win) {
         const uint64_t row_step = (uint64_t)S_kv * kLcgMul;
         const uint32_t thr = p.c.drop_threshold;
         floatx16 dv[DV / 32];
+        auto pass = [&](auto inf) {
+            constexpr bool INF = decltype(inf)::value;
+            if constexpr (INF) stage_first(inf);
 #pragma unroll
-        for (int dt = 0; dt < DV / 32; ++dt) dv[dt] = floatx16{};
-        __syncthreads();
-        for (int qb = qb0; qb < nqb; ++qb) {
-            const int q0 = qb * BQ;
-            const uint32_t qs = (uint32_t)(((qb - qb0) & 1) * Cfg::STAGE), os = qs + (uint32_t)QT::BYTES;
-            const bool on = live(q0);
-            floatx16 s = floatx16{};
-            if (on) {
+            for (int dt = 0; dt < DV / 32; ++dt) dv[dt] = floatx16{};
+            __syncthreads();
+            for (int qb = qb0; qb < nqb; ++qb) {
+                const int q0 = qb * BQ;
+                const uint32_t qs = (uint32_t)(((qb - qb0) & 1) * Cfg::STAGE), os = qs + (uint32_t)QT::BYTES;
+                const bool on = live(q0);
+                floatx16 s = floatx16{};
+                if (on) {
 #pragma unroll
-                for (int ks = 0; ks < DQK / 16; ++ks) s = mfma_bf3(QT::row(qs + swQ.row, ks, 0), k[ks], s);
-                const float* Fs = reinterpret_cast<const float*>(smem + os + OT::BYTES);
-                if (kw0 + 31 >= S_kv || (causal && q0 < kw0 + 31)) {
+                    for (int ks = 0; ks < DQK / 16; ++ks) s = mfma_bf3(QT::row(qs + swQ.row, ks, 0), k[ks], s);
+                    const float* Fs = reinterpret_cast<const float*>(smem + os + OT::BYTES);
+                    if (kw0 + 31 >= S_kv || (causal && q0 < kw0 + 31)) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int q = q0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-                        if (!key_ok || (causal && my_k > q)) s[r] = sl2 < 0.f ? INFINITY : -INFINITY;
-                    }
-                }
-                float sum = 0.f;
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const floatx4 st4 = *reinterpret_cast<const floatx4*>(Fs + 8 * g + 4 * hh);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        s[4 * g + e] = fast_exp2(__builtin_fmaf(s[4 * g + e], sl2, -st4[e]));
-                        sum += s[4 * g + e];
-                    }
-                }
-                if (wave_any(sum != sum)) {  // scores of -inf (see sdpa_f32_fwd.hip)
-                    floatx16 h = floatx16{};
-#pragma unroll
-                    for (int ks = 0; ks < DQK / 16; ++ks) h = mfma_bf16(QT::row(qs + swQ.row, ks, 0).p[0], k[ks].p[0], h);
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        if (h[r] * sl2 == -INFINITY) s[r] = 0.f;
-                }
-                const uint64_t st_blk = DROP ? st_base + (uint64_t)q0 * row_step : 0;
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    floatx4 xv;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float p0 = s[4 * g + e] > kEps ? s[4 * g + e] : 0.f;
-                        if constexpr (DROP) {
-                            const bool keep = lcg_keep(st_blk + (uint64_t)(8 * g + e) * row_step, thr);
-                            s[4 * g + e] = keep ? p0 : 0.f;
-                            xv[e] = keep ? p0 : -p0;
-                        } else {
-                            s[4 * g + e] = p0;
-                            xv[e] = p0;
+                        for (int r = 0; r < 16; ++r) {
+                            const int q = q0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+                            if (!key_ok || (causal && my_k > q)) s[r] = sl2 < 0.f ? INFINITY : -INFINITY;
                         }
                     }
-                    *reinterpret_cast<floatx4*>(xs + (g * 64 + lane) * 4) = xv;
-                }
-            }
-            __syncthreads();
-            if (on) {
+                    float sum = 0.f;
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const Bf3 pb = cut8([&](int i) { return s[8 * j + i]; });
+                    for (int g = 0; g < 4; ++g) {
+                        const floatx4 st4 = *reinterpret_cast<const floatx4*>(Fs + 8 * g + 4 * hh);
 #pragma unroll
-                    for (int dt = 0; dt < DV / 32; ++dt)
-                        dv[dt] = mfma_bf3(OT::tr(os + swO.tr0, os + swO.tr1, dt, 16 * j), pb, dv[dt]);
+                        for (int e = 0; e < 4; ++e) {
+                            s[4 * g + e] = fast_exp2(__builtin_fmaf(s[4 * g + e], sl2, -st4[e]));
+                            sum += s[4 * g + e];
+                        }
+                    }
+                    if (wave_any(sum != sum)) {  // scores of -inf (see sdpa_f32_fwd.hip)
+                        lds_read_again();
+                        floatx16 h = floatx16{};
+#pragma unroll
+                        for (int ks = 0; ks < DQK / 16; ++ks) h = mfma_bf16(QT::row(qs + swQ.row, ks, 0).p[0], k[ks].p[0], h);
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            if (h[r] * sl2 == -INFINITY) s[r] = 0.f;
+                    }
+                    const uint64_t st_blk = DROP ? st_base + (uint64_t)q0 * row_step : 0;
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        floatx4 xv;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float p0 = s[4 * g + e] > kEps ? s[4 * g + e] : 0.f;
+                            if constexpr (DROP) {
+                                const bool keep = lcg_keep(st_blk + (uint64_t)(8 * g + e) * row_step, thr);
+                                s[4 * g + e] = keep ? p0 : 0.f;
+                                xv[e] = keep ? p0 : -p0;
+                            } else {
+                                s[4 * g + e] = p0;
+                                xv[e] = p0;
+                            }
+                        }
+                        *reinterpret_cast<floatx4*>(xs + (g * 64 + lane) * 4) = xv;
+                    }
                 }
+                __syncthreads();
+                if (on) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const Bf3 pb = cut8([&](int i) { return s[8 * j + i]; });
+#pragma unroll
+                        for (int dt = 0; dt < DV / 32; ++dt)
+                            dv[dt] = mfma_bf3<INF>(OT::tr(os + swO.tr0, os + swO.tr1, dt, 16 * j), pb, dv[dt]);
+                    }
+                }
+                stage_next(qb, inf);
+                __syncthreads();
             }
-            stage_next(qb);
-            __syncthreads();
-        }
+        };
+        pass(std::false_type{});
+        if (workgroup_any_nan<Cfg::NT / 64>(dv, tid)) pass(std::true_type{});
         if (key_ok && np > 1)
             store_rows_f32<DV, VEC>(p.part_dv + ((size_t)(part * B + b) * S_kv + my_k) * D_v, dv, 1.f, hh, D_v);
         else if (key_ok)
@@ -196,63 +209,69 @@ void sdpa_bwd_dkdv_f32_bf3_kernel(const BwdParams p, const int win) {
         load_row_bf3<DV, VEC>(v, static_cast<const float*>(p.v) + (size_t)b * S_kv * D_v, my_k, S_kv, D_v, hh);
         const float ksc = p.c.keep_scale;
         floatx16 dk[DQK / 32];
-#pragma unroll
-        for (int dt = 0; dt < DQK / 32; ++dt) dk[dt] = floatx16{};
         const DsLayout32 dsl(S_q, S_kv, causal);
-        __syncthreads();
-        for (int qb = qb0; qb < nqb; ++qb) {
-            const int q0 = qb * BQ;
-            const uint32_t qs = (uint32_t)(((qb - qb0) & 1) * Cfg::STAGE), os = qs + (uint32_t)QT::BYTES;
-            const bool on = live(q0);
-            floatx16 dp = floatx16{};
-            if (on) {
+        auto pass = [&](auto inf) {
+            constexpr bool INF = decltype(inf)::value;
+            if constexpr (INF) stage_first(inf);
 #pragma unroll
-                for (int ks = 0; ks < DV / 16; ++ks) dp = mfma_bf3(OT::row(os + swO.row, ks, 0), v[ks], dp);
-            }
-            stage_next(qb);
+            for (int dt = 0; dt < DQK / 32; ++dt) dk[dt] = floatx16{};
             __syncthreads();
-            if (on) {
-                // dS = P0 (keep ? dP / (1-p) : 0 - delta), P0 = |x|, keep = x > 0
-                const float* Fs = reinterpret_cast<const float*>(smem + os + OT::BYTES);
+            for (int qb = qb0; qb < nqb; ++qb) {
+                const int q0 = qb * BQ;
+                const uint32_t qs = (uint32_t)(((qb - qb0) & 1) * Cfg::STAGE), os = qs + (uint32_t)QT::BYTES;
+                const bool on = live(q0);
+                floatx16 dp = floatx16{};
+                if (on) {
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const floatx4 xv = *reinterpret_cast<const floatx4*>(xs + (g * 64 + lane) * 4);
-                    const floatx4 de4 = *reinterpret_cast<const floatx4*>(Fs + BQ + 8 * g + 4 * hh);
+                    for (int ks = 0; ks < DV / 16; ++ks) dp = mfma_bf3<INF>(OT::row(os + swO.row, ks, 0), v[ks], dp);
+                }
+                stage_next(qb, inf);
+                __syncthreads();
+                if (on) {
+                    // dS = P0 (keep ? dP / (1-p) : 0 - delta), P0 = |x|, keep = x > 0
+                    const float* Fs = reinterpret_cast<const float*>(smem + os + OT::BYTES);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float d = DROP ? dp[4 * g + e] * ksc : dp[4 * g + e];
-                        float p0 = xv[e];
-                        if constexpr (DROP) {
-                            d = xv[e] > 0.f ? d : 0.f;
-                            p0 = __builtin_fabsf(xv[e]);
+                    for (int g = 0; g < 4; ++g) {
+                        const floatx4 xv = *reinterpret_cast<const floatx4*>(xs + (g * 64 + lane) * 4);
+                        const floatx4 de4 = *reinterpret_cast<const floatx4*>(Fs + BQ + 8 * g + 4 * hh);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            float d = DROP ? dp[4 * g + e] * ksc : dp[4 * g + e];
+                            float p0 = xv[e];
+                            if constexpr (DROP) {
+                                d = xv[e] > 0.f ? d : 0.f;
+                                p0 = __builtin_fabsf(xv[e]);
+                            }
+                            dp[4 * g + e] = p0 * (d - de4[e]);
                         }
-                        dp[4 * g + e] = p0 * (d - de4[e]);
+                    }
+                    if constexpr (DS) {
+                        // the lane's 16 values as four 16-byte slots of its key
+                        // group (DsLayout32), each store 1 KB whole, non-temporal;
+                        // zero for keys past S_kv (dQ reads them unmasked)
+                        unsigned char* grp = static_cast<unsigned char*>(p.ds) + dsl.offset(b, kt, qb) + kw * 4096;
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            floatx4 x;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) x[e] = key_ok ? dp[4 * u + e] : 0.f;
+                            __builtin_nontemporal_store(
+                                x, reinterpret_cast<floatx4*>(grp + DsLayout32::slot32(l32, 16 * hh + 4 * u)));
+                        }
+                    }
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const Bf3 db = cut8<INF>([&](int i) { return dp[8 * j + i]; });
+#pragma unroll
+                        for (int dt = 0; dt < DQK / 32; ++dt)
+                            dk[dt] = mfma_bf3<INF>(QT::tr(qs + swQ.tr0, qs + swQ.tr1, dt, 16 * j), db, dk[dt]);
                     }
                 }
-                if constexpr (DS) {
-                    // the lane's 16 values as four 16-byte slots of its key
-                    // group (DsLayout32), each store 1 KB whole, non-temporal;
-                    // zero for keys past S_kv (dQ reads them unmasked)
-                    unsigned char* grp = static_cast<unsigned char*>(p.ds) + dsl.offset(b, kt, qb) + kw * 4096;
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        floatx4 x;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) x[e] = key_ok ? dp[4 * u + e] : 0.f;
-                        __builtin_nontemporal_store(
-                            x, reinterpret_cast<floatx4*>(grp + DsLayout32::slot32(l32, 16 * hh + 4 * u)));
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const Bf3 db = cut8([&](int i) { return dp[8 * j + i]; });
-#pragma unroll
-                    for (int dt = 0; dt < DQK / 32; ++dt)
-                        dk[dt] = mfma_bf3(QT::tr(qs + swQ.tr0, qs + swQ.tr1, dt, 16 * j), db, dk[dt]);
-                }
+                __syncthreads();
             }
-            __syncthreads();
-        }
+        };
+        pass(std::false_type{});
+        if (workgroup_any_nan<Cfg::NT / 64>(dk, tid)) pass(std::true_type{});
         if (key_ok && np > 1)
             store_rows_f32<DQK, VEC>(p.part_dk + ((size_t)(part * B + b) * S_kv + my_k) * D_qk, dk, 1.f, hh, D_qk);
         else if (key_ok)

@@ -88,8 +88,6 @@ void sdpa_bwd_dq_f32_bf3_kernel(const BwdParams p, const int win) {
     swK.init(lane);
     swV.init(lane);
     floatx16 dq[NDT];
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) dq[dt] = floatx16{};
 
     Bf3Stage<BN, DQK, Cfg::NT, VEC> kst;
     Bf3Stage<BN, DV, Cfg::NT, VEC> vst;
@@ -98,71 +96,80 @@ void sdpa_bwd_dq_f32_bf3_kernel(const BwdParams p, const int win) {
         kst.load(Kb, n0, S_kv - n0, D_qk, D_qk, tid);
         vst.load(Vb, n0, S_kv - n0, D_v, D_v, tid);
     };
-    auto store_block = [&](int blk) {
-        unsigned char* n = smem + ((blk - lo) & 1) * Cfg::STAGE;
-        kst.store(n, tid);
-        vst.store(n + KT::BYTES, tid);
-    };
-    if (lo < hi) {
-        load_block(lo);
-        store_block(lo);
-        if (lo + 1 < hi) load_block(lo + 1);
-    }
-    __syncthreads();
-
-    for (int blk = lo; blk < hi; ++blk) {
-        const int kv0 = blk * BN + 32 * wk;
-        const uint32_t ks0 = (uint32_t)(((blk - lo) & 1) * Cfg::STAGE), vs0 = ks0 + (uint32_t)KT::BYTES;
-        if (wave_live && kv0 < S_kv && (!causal || kv0 <= wave_last_q)) {
-            floatx16 s = floatx16{}, dp = floatx16{};
+    // INF: again, for infinities in V, dO or dS (sdpa_bf3.h)
+    auto pass = [&](auto inf) {
+        constexpr bool INF = decltype(inf)::value;
 #pragma unroll
-            for (int ks = 0; ks < DQK / 16; ++ks) s = mfma_bf3(KT::row(ks0 + swK.row, ks, 32 * wk), q[ks], s);
-#pragma unroll
-            for (int ks = 0; ks < DV / 16; ++ks) dp = mfma_bf3(VT::row(vs0 + swV.row, ks, 32 * wk), d_o[ks], dp);
-            float sum = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[r] = fast_exp2(__builtin_fmaf(s[r], sl2, -stats2));
-                sum += s[r];
-            }
-            if (wave_any(sum != sum)) {  // scores of -inf (see sdpa_f32_fwd.hip)
-                floatx16 h = floatx16{};
-#pragma unroll
-                for (int ks = 0; ks < DQK / 16; ++ks)
-                    h = mfma_bf16(KT::row(ks0 + swK.row, ks, 32 * wk).p[0], q[ks].p[0], h);
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (h[r] * sl2 == -INFINITY) s[r] = 0.f;
-            }
-            if (kv0 + 32 > S_kv || (causal && kv0 + 31 > qw0)) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = kv0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-                    if (key >= S_kv || (causal && key > my_q)) s[r] = 0.f;
-                }
-            }
-            const uint64_t st_blk = DROP ? st_base + (uint64_t)kv0 * kLcgMul : 0;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float p0 = s[r] > kEps ? s[r] : 0.f;
-                float d = DROP ? dp[r] * ksc : dp[r];
-                if constexpr (DROP) d = lcg_keep(st_blk + (uint64_t)(8 * (r >> 2) + (r & 3)) * kLcgMul, thr) ? d : 0.f;
-                dp[r] = p0 * (d - delta);
-            }
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const Bf3 ds = cut8([&](int i) { return dp[8 * j + i]; });
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt)
-                    dq[dt] = mfma_bf3(KT::tr(ks0 + swK.tr0, ks0 + swK.tr1, dt, 32 * wk + 16 * j), ds, dq[dt]);
-            }
-        }
-        if (blk + 1 < hi) {
-            store_block(blk + 1);
-            if (blk + 2 < hi) load_block(blk + 2);
+        for (int dt = 0; dt < NDT; ++dt) dq[dt] = floatx16{};
+        auto store_block = [&](int blk) {
+            unsigned char* n = smem + ((blk - lo) & 1) * Cfg::STAGE;
+            kst.store(n, tid);
+            vst.template store<INF>(n + KT::BYTES, tid);
+        };
+        if (lo < hi) {
+            load_block(lo);
+            store_block(lo);
+            if (lo + 1 < hi) load_block(lo + 1);
         }
         __syncthreads();
-    }
+
+        for (int blk = lo; blk < hi; ++blk) {
+            const int kv0 = blk * BN + 32 * wk;
+            const uint32_t ks0 = (uint32_t)(((blk - lo) & 1) * Cfg::STAGE), vs0 = ks0 + (uint32_t)KT::BYTES;
+            if (wave_live && kv0 < S_kv && (!causal || kv0 <= wave_last_q)) {
+                floatx16 s = floatx16{}, dp = floatx16{};
+#pragma unroll
+                for (int ks = 0; ks < DQK / 16; ++ks) s = mfma_bf3(KT::row(ks0 + swK.row, ks, 32 * wk), q[ks], s);
+#pragma unroll
+                for (int ks = 0; ks < DV / 16; ++ks) dp = mfma_bf3<INF>(VT::row(vs0 + swV.row, ks, 32 * wk), d_o[ks], dp);
+                float sum = 0.f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s[r] = fast_exp2(__builtin_fmaf(s[r], sl2, -stats2));
+                    sum += s[r];
+                }
+                if (wave_any(sum != sum)) {  // scores of -inf (see sdpa_f32_fwd.hip)
+                    lds_read_again();
+                    floatx16 h = floatx16{};
+#pragma unroll
+                    for (int ks = 0; ks < DQK / 16; ++ks)
+                        h = mfma_bf16(KT::row(ks0 + swK.row, ks, 32 * wk).p[0], q[ks].p[0], h);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (h[r] * sl2 == -INFINITY) s[r] = 0.f;
+                }
+                if (kv0 + 32 > S_kv || (causal && kv0 + 31 > qw0)) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int key = kv0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+                        if (key >= S_kv || (causal && key > my_q)) s[r] = 0.f;
+                    }
+                }
+                const uint64_t st_blk = DROP ? st_base + (uint64_t)kv0 * kLcgMul : 0;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float p0 = s[r] > kEps ? s[r] : 0.f;
+                    float d = DROP ? dp[r] * ksc : dp[r];
+                    if constexpr (DROP) d = lcg_keep(st_blk + (uint64_t)(8 * (r >> 2) + (r & 3)) * kLcgMul, thr) ? d : 0.f;
+                    dp[r] = p0 * (d - delta);
+                }
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const Bf3 ds = cut8<INF>([&](int i) { return dp[8 * j + i]; });
+#pragma unroll
+                    for (int dt = 0; dt < NDT; ++dt)
+                        dq[dt] = mfma_bf3<INF>(KT::tr(ks0 + swK.tr0, ks0 + swK.tr1, dt, 32 * wk + 16 * j), ds, dq[dt]);
+                }
+            }
+            if (blk + 1 < hi) {
+                store_block(blk + 1);
+                if (blk + 2 < hi) load_block(blk + 2);
+            }
+            __syncthreads();
+        }
+    };
+    pass(std::false_type{});
+    if (workgroup_any_nan<Cfg::NT / 64>(dq, tid)) pass(std::true_type{});
 
     // the second wave of each group through LDS
     float* m = reinterpret_cast<float*>(smem) + (32 * wq + l32) * Cfg::OS;

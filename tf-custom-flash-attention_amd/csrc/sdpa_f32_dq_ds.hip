@@ -128,38 +128,44 @@ void sdpa_bwd_dq_ds_f32_kernel(const BwdParams p, const int win) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) sbase[e] = DsLayout32::slot32(4 * hh + e, l32);
     floatx16 acc[NDT];
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) acc[dt] = floatx16{};
 
-    if (nsteps > 0) {
-        copy_ds(0);
-        load_k(0);
-        store_k(0);
-        wait_vm();
-        if (nsteps > 1) load_k(1);
-    }
-    __syncthreads();
-    for (int step = 0; step < nsteps; ++step) {
-        // the other stages were released at the last barrier
-        if (step + 1 < nsteps) copy_ds(step + 1);
-        if (live(step * BN + 32 * wk)) {
-            const uint32_t ks0 = (uint32_t)((step & 1) * KT::BYTES);
-            const unsigned char* Ss = smem + s0 + (step & 1) * Cfg::SB;
+    // INF: again, for infinities in dS (sdpa_bf3.h)
+    auto pass = [&](auto inf) {
+        constexpr bool INF = decltype(inf)::value;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const Bf3 ds = cut8([&](int i) {
-                    return *reinterpret_cast<const float*>(Ss + sbase[i & 3] + 128 * (2 * j + (i >> 2)));
-                });
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt)
-                    acc[dt] = mfma_bf3(KT::tr(ks0 + swK.tr0, ks0 + swK.tr1, dt, 32 * wk + 16 * j), ds, acc[dt]);
-            }
+        for (int dt = 0; dt < NDT; ++dt) acc[dt] = floatx16{};
+        if (nsteps > 0) {
+            copy_ds(0);
+            load_k(0);
+            store_k(0);
+            wait_vm();
+            if (nsteps > 1) load_k(1);
         }
-        if (step + 1 < nsteps) store_k(step + 1);
-        wait_vm();  // the next step's dS
-        if (step + 2 < nsteps) load_k(step + 2);
         __syncthreads();
-    }
+        for (int step = 0; step < nsteps; ++step) {
+            // the other stages were released at the last barrier
+            if (step + 1 < nsteps) copy_ds(step + 1);
+            if (live(step * BN + 32 * wk)) {
+                const uint32_t ks0 = (uint32_t)((step & 1) * KT::BYTES);
+                const unsigned char* Ss = smem + s0 + (step & 1) * Cfg::SB;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const Bf3 ds = cut8<INF>([&](int i) {
+                        return *reinterpret_cast<const float*>(Ss + sbase[i & 3] + 128 * (2 * j + (i >> 2)));
+                    });
+#pragma unroll
+                    for (int dt = 0; dt < NDT; ++dt)
+                        acc[dt] = mfma_bf3<INF>(KT::tr(ks0 + swK.tr0, ks0 + swK.tr1, dt, 32 * wk + 16 * j), ds, acc[dt]);
+                }
+            }
+            if (step + 1 < nsteps) store_k(step + 1);
+            wait_vm();  // the next step's dS
+            if (step + 2 < nsteps) load_k(step + 2);
+            __syncthreads();
+        }
+    };
+    pass(std::false_type{});
+    if (workgroup_any_nan<Cfg::NT / 64>(acc, tid)) pass(std::true_type{});
 
     float* m = reinterpret_cast<float*>(smem) + (32 * wq + l32) * Cfg::OS;
     if (wk == 1) store_rows_f32<DQK, true>(m, acc, 1.f, hh, DQK);

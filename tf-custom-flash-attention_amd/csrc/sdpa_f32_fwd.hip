@@ -88,9 +88,7 @@ void sdpa_fwd_f32_bf3_kernel(const FwdParams p, const int win) {
     const bool wave_live = qw0 < S_q;
     const int wave_last_q = min(qw0 + 31, S_q - 1);
     floatx16 oacc[NDT];
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) oacc[dt] = floatx16{};
-    float m_run = kMaxSentinel, l_run = 0.f;
+    float m_run, l_run;
     const uint64_t st_base = DROP ? lcg_state(p.c.seed_offset, (uint64_t)b * S_q + my_q, (uint64_t)S_kv, 4 * hh) : 0;
     const uint32_t thr = p.c.drop_threshold;
     SwzLane<LK> swK;
@@ -105,99 +103,115 @@ void sdpa_fwd_f32_bf3_kernel(const FwdParams p, const int win) {
         kst.load(Kb, n0, S_kv - n0, D_qk, D_qk, tid);
         vst.load(Vb, n0, S_kv - n0, D_v, D_v, tid);
     };
-    auto store_block = [&](int blk) {
-        unsigned char* n = smem + ((blk - lo) & 1) * Cfg::STAGE;
-        kst.store(n, tid);
-        vst.store(n + KT::BYTES, tid);
-    };
-    if (lo < hi) {
-        load_block(lo);
-        store_block(lo);
-        if (lo + 1 < hi) load_block(lo + 1);
-    }
-    __syncthreads();
-
-    // The registers hold block blk + 1; it goes to LDS, and block blk + 2 into
-    // the registers, at the end of the step.
-    for (int blk = lo; blk < hi; ++blk) {
-        const int kv0 = blk * BN + 32 * wk;
-        const uint32_t ks0 = (uint32_t)(((blk - lo) & 1) * Cfg::STAGE), vs0 = ks0 + (uint32_t)KT::BYTES;
-        if (wave_live && kv0 < S_kv && (!causal || kv0 <= wave_last_q)) {
-            floatx16 s = floatx16{};
+    // INF: again, for infinities in V (sdpa_bf3.h)
+    auto pass = [&](auto inf) {
+        constexpr bool INF = decltype(inf)::value;
 #pragma unroll
-            for (int ks = 0; ks < DQK / 16; ++ks) s = mfma_bf3(KT::row(ks0 + swK.row, ks, 32 * wk), q[ks], s);
-            if ((kv0 + 32 > S_kv) || (causal && kv0 + 31 > qw0)) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = kv0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-                    if (key >= S_kv || (causal && key > my_q)) s[r] = -INFINITY;
-                }
-            }
-            float mx = fmaxf(fmaxf(s[0], s[1]), s[2]);
-#pragma unroll
-            for (int r = 3; r < 15; r += 2) {
-                mx = fmaxf(mx, fmaxf(s[r], s[r + 1]));
-            }
-            mx = xhalf_max(fmaxf(mx, s[15])) * sl2;
-            const float m_new = fmaxf(m_run, mx);
-            if (wave_any(m_new > m_run + kTau32)) {
-                const float alpha = fast_exp2(m_run - m_new);
-                l_run *= alpha;
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
-                m_run = m_new;
-            }
-            const uint64_t st_blk = DROP ? st_base + (uint64_t)kv0 * kLcgMul : 0;
-            float lsum = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[r] = fast_exp2(__builtin_fmaf(s[r], sl2, -m_run));
-                lsum += s[r];
-            }
-            if (wave_any(lsum != lsum)) {
-                // A score of -inf (an infinite q or k) reads NaN in the sum of
-                // the parts' products, -inf in that of the first parts alone.
-                floatx16 h = floatx16{};
-#pragma unroll
-                for (int ks = 0; ks < DQK / 16; ++ks)
-                    h = mfma_bf16(KT::row(ks0 + swK.row, ks, 32 * wk).p[0], q[ks].p[0], h);
-                lsum = 0.f;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    if (h[r] == -INFINITY) s[r] = 0.f;
-                    lsum += s[r];
-                }
-            }
-            if constexpr (DROP) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (!lcg_keep(st_blk + (uint64_t)(8 * (r >> 2) + (r & 3)) * kLcgMul, thr)) s[r] = 0.f;
-            }
-            l_run += lsum;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const Bf3 pb = cut8([&](int i) { return s[8 * j + i]; });
-                Bf3 va[NDT];
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt) va[dt] = VT::tr(vs0 + swV.tr0, vs0 + swV.tr1, dt, 32 * wk + 16 * j);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < 6; ++i)
-#pragma unroll
-                    for (int dt = 0; dt < NDT; ++dt) {
-                        constexpr int ia[6] = {2, 0, 1, 1, 0, 0}, ib[6] = {0, 2, 1, 0, 1, 0};
-                        oacc[dt] = mfma_bf16(va[dt].p[ia[i]], pb.p[ib[i]], oacc[dt]);
-                    }
-            }
-        }
-        if (blk + 1 < hi) {
-            store_block(blk + 1);
-            if (blk + 2 < hi) load_block(blk + 2);
+        for (int dt = 0; dt < NDT; ++dt) oacc[dt] = floatx16{};
+        m_run = kMaxSentinel;
+        l_run = 0.f;
+        auto store_block = [&](int blk) {
+            unsigned char* n = smem + ((blk - lo) & 1) * Cfg::STAGE;
+            kst.store(n, tid);
+            vst.template store<INF>(n + KT::BYTES, tid);
+        };
+        if (lo < hi) {
+            load_block(lo);
+            store_block(lo);
+            if (lo + 1 < hi) load_block(lo + 1);
         }
         __syncthreads();
-    }
+
+        // The registers hold block blk + 1; it goes to LDS, and block blk + 2 into
+        // the registers, at the end of the step.
+        for (int blk = lo; blk < hi; ++blk) {
+            const int kv0 = blk * BN + 32 * wk;
+            const uint32_t ks0 = (uint32_t)(((blk - lo) & 1) * Cfg::STAGE), vs0 = ks0 + (uint32_t)KT::BYTES;
+            if (wave_live && kv0 < S_kv && (!causal || kv0 <= wave_last_q)) {
+                floatx16 s = floatx16{};
+#pragma unroll
+                for (int ks = 0; ks < DQK / 16; ++ks) s = mfma_bf3(KT::row(ks0 + swK.row, ks, 32 * wk), q[ks], s);
+                if ((kv0 + 32 > S_kv) || (causal && kv0 + 31 > qw0)) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int key = kv0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+                        if (key >= S_kv || (causal && key > my_q)) s[r] = -INFINITY;
+                    }
+                }
+                float mx = fmaxf(fmaxf(s[0], s[1]), s[2]);
+#pragma unroll
+                for (int r = 3; r < 15; r += 2) {
+                    mx = fmaxf(mx, fmaxf(s[r], s[r + 1]));
+                }
+                mx = xhalf_max(fmaxf(mx, s[15])) * sl2;
+                const float m_new = fmaxf(m_run, mx);
+                if (wave_any(m_new > m_run + kTau32)) {
+                    const float alpha = fast_exp2(m_run - m_new);
+                    l_run *= alpha;
+#pragma unroll
+                    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+                    m_run = m_new;
+                }
+                const uint64_t st_blk = DROP ? st_base + (uint64_t)kv0 * kLcgMul : 0;
+                float lsum = 0.f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s[r] = fast_exp2(__builtin_fmaf(s[r], sl2, -m_run));
+                    lsum += s[r];
+                }
+                if (wave_any(lsum != lsum)) {
+                    // A score of -inf (an infinite q or k) reads NaN in the sum of
+                    // the parts' products, -inf in that of the first parts alone.
+                    lds_read_again();
+                    floatx16 h = floatx16{};
+#pragma unroll
+                    for (int ks = 0; ks < DQK / 16; ++ks)
+                        h = mfma_bf16(KT::row(ks0 + swK.row, ks, 32 * wk).p[0], q[ks].p[0], h);
+                    lsum = 0.f;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        if (h[r] == -INFINITY) s[r] = 0.f;
+                        lsum += s[r];
+                    }
+                }
+                if constexpr (DROP) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (!lcg_keep(st_blk + (uint64_t)(8 * (r >> 2) + (r & 3)) * kLcgMul, thr)) s[r] = 0.f;
+                }
+                l_run += lsum;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const Bf3 pb = cut8([&](int i) { return s[8 * j + i]; });
+                    Bf3 va[NDT];
+#pragma unroll
+                    for (int dt = 0; dt < NDT; ++dt) va[dt] = VT::tr(vs0 + swV.tr0, vs0 + swV.tr1, dt, 32 * wk + 16 * j);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (INF) {
+#pragma unroll
+                        for (int dt = 0; dt < NDT; ++dt) oacc[dt] = mfma_bf3<true>(va[dt], pb, oacc[dt]);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 6; ++i)
+#pragma unroll
+                            for (int dt = 0; dt < NDT; ++dt) {
+                                constexpr int ia[6] = {2, 0, 1, 1, 0, 0}, ib[6] = {0, 2, 1, 0, 1, 0};
+                                oacc[dt] = mfma_bf16(va[dt].p[ia[i]], pb.p[ib[i]], oacc[dt]);
+                            }
+                    }
+                }
+            }
+            if (blk + 1 < hi) {
+                store_block(blk + 1);
+                if (blk + 2 < hi) load_block(blk + 2);
+            }
+            __syncthreads();
+        }
+    };
+    pass(std::false_type{});
+    if (workgroup_any_nan<Cfg::NT / 64>(oacc, tid)) pass(std::true_type{});
 
     float l_tot = xhalf_sum(l_run);
     if constexpr (Cfg::NWK == 2) {
