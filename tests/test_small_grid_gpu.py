@@ -318,6 +318,8 @@ BWD = [
     ("f32", 2, 160, 160, 128, 128, True, 0.2, 1),   # dS path
     ("f32", 1, 31, 257, 128, 32, False, 1.5, 1),    # dS path, every element dropped
     ("f32", 1, 17, 8193, 40, 36, False, 0.1, 1),    # the sequential fp32 sums, undivided
+    ("f32", 2, 5, 8200, 64, 64, False, 0.1, 2),     # the same for few queries, dQ in parts
+    ("f32", 1, 16, 9001, 37, 5, False, 0.0, 2),     # and with element loads
     ("f32", 1, 33, 8225, 128, 64, False, 0.0, 1),   # the same, dS path
 ]
 

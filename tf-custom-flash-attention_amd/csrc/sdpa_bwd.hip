@@ -515,9 +515,10 @@ void sdpa_bwd_dq_f32_kernel(const BwdParams p) {
     const int l32 = lane & 31, hh = lane >> 5;
     const int B = p.s.B, S_q = p.s.S_q, S_kv = p.s.S_kv, D_qk = p.s.D_qk, D_v = p.s.D_v;
     const bool causal = p.c.causal != 0;
-    const int tiles = (S_q + BM - 1) / BM;
-    int b, qt;
-    map_tile(blockIdx.x, B, tiles, causal, b, qt);
+    const int np = p.parts, items = (S_q + BM - 1) / BM * np;
+    int b, it;
+    map_tile(blockIdx.x, B, items, causal, b, it);
+    const int qt = it / np, part = it - qt * np;
     const int q0 = qt * BM, qw0 = q0 + wave * 32, my_q = qw0 + l32;
     const size_t row_q = (size_t)b * S_q + my_q;
 
@@ -548,7 +549,7 @@ void sdpa_bwd_dq_f32_kernel(const BwdParams p) {
     const float delta = xhalf_sum(dpart);
     const bool row_ok = my_q < S_q;
     const float stats2 = row_ok ? p.stats[row_q] * kLog2e : INFINITY;
-    if (row_ok && hh == 0) {
+    if (row_ok && hh == 0 && part == 0) {
         p.delta[row_q] = delta;
         p.stats2[row_q] = stats2 + kGateShift;
     }
@@ -556,7 +557,8 @@ void sdpa_bwd_dq_f32_kernel(const BwdParams p) {
     const float ksc = p.c.keep_scale;
 
     const int kv_end = causal ? min(S_kv, q0 + BM) : S_kv;
-    const int nblk = (kv_end + BN - 1) / BN;
+    const int blocks = (kv_end + BN - 1) / BN;  // of them this part's: [lo, nblk)
+    const int lo = part_begin(blocks, part, np), nblk = part_begin(blocks, part + 1, np);
     const bool wave_live = qw0 < S_q;
     const int wave_last_q = min(qw0 + 31, S_q - 1);
     const uint64_t st_base = DROP ? lcg_state(p.c.seed_offset, row_q, (uint64_t)S_kv, 4 * hh) : 0;
@@ -568,15 +570,16 @@ void sdpa_bwd_dq_f32_kernel(const BwdParams p) {
 
     TileStage<float, BN, DQK, Cfg::NT, VEC> kst;
     TileStage<float, BN, DV, Cfg::NT, VEC> vst;
-    if (nblk > 0) {
-        kst.load(Kb, 0, S_kv, D_qk, D_qk, tid);
-        vst.load(Vb, 0, S_kv, D_v, D_v, tid);
-        kst.template store<KS>(lds, tid);
-        vst.template store<VS>(lds + Cfg::KT, tid);
+    if (lo < nblk) {
+        float* K0 = lds + (lo & 1) * Cfg::STAGE;
+        kst.load(Kb, lo * BN, S_kv - lo * BN, D_qk, D_qk, tid);
+        vst.load(Vb, lo * BN, S_kv - lo * BN, D_v, D_v, tid);
+        kst.template store<KS>(K0, tid);
+        vst.template store<VS>(K0 + Cfg::KT, tid);
     }
     __syncthreads();
 
-    for (int blk = 0; blk < nblk; ++blk) {
+    for (int blk = lo; blk < nblk; ++blk) {
         const int kv0 = blk * BN;
         const float* Ks = lds + (blk & 1) * Cfg::STAGE;
         const float* Vs = Ks + Cfg::KT;
@@ -640,8 +643,8 @@ void sdpa_bwd_dq_f32_kernel(const BwdParams p) {
     }
 
     if (row_ok) {
-        const float sc = p.c.scale;
-        float* dQb = static_cast<float*>(p.dq) + row_q * D_qk;
+        const float sc = np > 1 ? 1.f : p.c.scale;
+        float* dQb = np > 1 ? p.part_dq + ((size_t)part * B * S_q + row_q) * D_qk : static_cast<float*>(p.dq) + row_q * D_qk;
 #pragma unroll
         for (int dt = 0; dt < DQK / 32; ++dt)
 #pragma unroll
@@ -693,7 +696,7 @@ hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, bool half4, int
                         if (phases & kBwdDq) {
                             if (DQK == 128 || DV == 128 || fp32_chain(p.s)) {
                                 using CQ = BwdQF32Cfg<DQK, DV>;
-                                const unsigned gq = (unsigned)(((S_q + CQ::BM - 1) / CQ::BM) * B);
+                                const unsigned gq = (unsigned)(((S_q + CQ::BM - 1) / CQ::BM) * p.parts * B);
                                 err = launch_kernel<sdpa_bwd_dq_f32_kernel<DQK, DV, V, D>>(gq, CQ::NT, CQ::LDS_BYTES, stream, p);
                             } else {
                                 err = launch_bwd_dq_f32(p, V, stream);

@@ -62,8 +62,14 @@ inline int pad_dim(int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }
 // the gate of the gradient lies among the weights of ordinary rows (figures
 // there: none of 40 calls differed up to 12000 keys, 11 of 38 at 16384; for
 // scores of unit variance the weights near the gate grow 16-fold from 8192 to
-// 16384 keys).  Up to 16 queries are generation, which takes no gradient.
-inline bool fp32_chain(const AttnShape& s) { return s.S_kv > 8192 && s.S_q > 16; }
+// 16384 keys).  The gradient's kernels go by the keys alone: given q, k and
+// stats, a weight keeps its side.  The forward of up to 16 queries (generation)
+// divides its keys on the bf16 matrix cores; its stats, 2e-6 from the chain's
+// at most, moved a weight in 0, 2 and 11 of 20 calls at B 64, S_q 16, S_kv
+// 16384, D 64 and 128, and S_q 4, S_kv 32768 (with the gradient there as well
+// 3, 7 and 20; the largest change of an element 7e-4 of the root mean square).
+inline bool fp32_chain(const AttnShape& s) { return s.S_kv > 8192; }
+inline bool fp32_chain_fwd(const AttnShape& s) { return fp32_chain(s) && s.S_q > 16; }
 
 // Parts of the keys of a 128-query tile in the fp32 forward (sdpa_f32_fwd.hip).
 // A block (64 keys, 32 where both sides are 128 wide) takes about 0.0215 us
@@ -72,7 +78,7 @@ inline bool fp32_chain(const AttnShape& s) { return s.S_kv > 8192 && s.S_q > 16;
 // S_kv 8000, D 64: 288 -> 22.6 (32 parts); B 64, S_q 64, S_kv 2000, D 128:
 // 194 -> 65 (4); B 24, S 700, D 64: 38 (1; in two parts 57: a second round).
 inline int fwd_f32_parts(int B, int S_q, int S_kv, int D_qk, int D_v, bool causal) {
-    if (fp32_chain(AttnShape{B, S_q, S_kv, D_qk, D_v})) return 1;
+    if (fp32_chain_fwd(AttnShape{B, S_q, S_kv, D_qk, D_v})) return 1;
     const int pq = pad_dim(D_qk), pv = pad_dim(D_v);
     const bool wide = pq == 128 && pv == 128;
     return least_time_parts((long long)B * ((S_q + 127) / 128), ((long long)S_kv + (wide ? 31 : 63)) / (wide ? 32 : 64),
@@ -230,6 +236,15 @@ inline BwdParts bwd_parts(bool f16, const AttnShape& s, bool causal) {
         r.kv = least_time_parts((long long)s.B * ((s.S_kv + 127) / 128), ((long long)s.S_q + 31) / 32, causal,
                                 0.8 + 0.0085 * cols, 3, 8.0 * s.B * s.S_kv * (s.D_qk + s.D_v));
     }
+    if (!f16 && fp32_chain(s) && s.S_q <= 16)
+        // Blocks of 32 keys of the sequential sums (3.5 us at D = 64), for the
+        // few queries whose forward divides too; the gate does not see the
+        // division.  Undivided -> chosen, us of the whole backward at D = 64: B
+        // 64, S_q 16, S_kv 16384: 2237 -> 866; B 16, S_q 8, S_kv 12000: 1468 ->
+        // 177; B 1, S_q 16, S_kv 65536: 7299 -> 164 (on the bf16 matrix cores
+        // 536, 113 and 91).
+        r.q = least_time_parts(s.B, ((long long)s.S_kv + 31) / 32, causal,
+                               0.036 * (pad_dim(s.D_qk) + 0.5 * pad_dim(s.D_v)), 3, 8.0 * s.B * s.S_q * s.D_qk);
     if (r.q > 1) r.dq_floats = (size_t)r.q * s.B * s.S_q * s.D_qk;
     if (r.kv > 1) {
         r.dk_floats = (size_t)r.kv * s.B * s.S_kv * s.D_qk;
