@@ -124,6 +124,30 @@ def test_f32_grid_of_more_threads_than_one_dimension(pkg):
     assert dq.abs().max().item() <= 1e-4 and dk.abs().max().item() <= 1e-4
 
 
+@pytest.mark.parametrize("dtype,D", [(torch.float16, 64), (torch.float32, 64), (torch.float16, 128)])
+def test_workspace_that_cannot_be_had(pkg, monkeypatch, dtype, D):
+    """Calls whose tiles would be divided, or whose dS stored, run undivided
+    where the memory for it is not there."""
+    g = torch.Generator().manual_seed(11)
+    q, k, v, d_o = (torch.randn((2, n, D), generator=g).to(dtype).cuda() for n in (16, 3000, 3000, 16))
+    o, s = pkg.sdpa(q, k, v, scale=0.1)
+    want = (o, s) + pkg.sdpa_grad(q, k, v, o, s, d_o, scale=0.1)
+    empty, refused, rows = torch.empty, [], pkg.library().sdpa_hip_bwd_workspace_bytes(2, 16)
+
+    def no_room(size, **kw):
+        if kw.get("dtype") is torch.uint8 and size[0] > rows:
+            refused.append(size[0])
+            raise torch.OutOfMemoryError("no room")
+        return empty(size, **kw)
+
+    monkeypatch.setattr(torch, "empty", no_room)
+    got = pkg.sdpa(q, k, v, scale=0.1) + pkg.sdpa_grad(q, k, v, o, s, d_o, scale=0.1)
+    assert len(refused) == 2
+    tol = TOL["f16" if dtype == torch.float16 else "f32"]
+    for name, a, b in zip(("o", "stats", "grad", "grad", "grad"), got, want):
+        assert (a.float() - b.float()).abs().max().item() <= tol[name] * max(1.0, b.float().abs().max().item())
+
+
 def test_half4_neighbour_row(pkg):
     """An infinity in a row does not reach the row before it, whose last chunk
     is copied with the first features of that one."""

@@ -194,6 +194,15 @@ def _plain_fwd(torch, q, k, v, seed, offset, causal_mask) -> bool:
             and sv[1] == sk[1] and sq[2] <= 128 and sv[2] <= 128 and (not causal_mask or sq[1] == sk[1]))
 
 
+def _workspace(torch, nbytes: int, device):
+    """``nbytes`` of device memory, None where those cannot be had: the call
+    then does with the least, as in the TensorFlow op."""
+    try:
+        return torch.empty((nbytes,), dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def sdpa(q, k, v, seed=0, offset=0, dropout: float = 0.0, scale: float = 1.0,
          causal_mask: bool = False):
     """Forward op ``Sdpa`` (sdpa_ops.cc:7-32): returns ``(o, stats)``.
@@ -215,7 +224,9 @@ def sdpa(q, k, v, seed=0, offset=0, dropout: float = 0.0, scale: float = 1.0,
     stats = torch.empty((B, S_q), dtype=torch.float32, device=q.device)
     L = library()
     ws_bytes = L.sdpa_hip_fwd_workspace_bytes(dt, B, S_q, S_kv, D_qk, D_v, int(bool(causal_mask)))
-    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=q.device) if ws_bytes else None
+    ws = _workspace(torch, ws_bytes, q.device) if ws_bytes else None
+    if ws is None:
+        ws_bytes = 0
     rc = L.sdpa_hip_fwd_ws(dt, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), stats.data_ptr(),
                            ws.data_ptr() if ws_bytes else None, ws_bytes, B, S_q, S_kv, D_qk, D_v,
                            float(scale), float(dropout), int(bool(causal_mask)), _u64(seed), _u64(offset),
@@ -251,12 +262,14 @@ def sdpa_grad(q, k, v, o, stats, d_o, seed=0, offset=0, dropout: float = 0.0,
     dq = torch.empty_like(q)
     dk = torch.empty_like(k)
     dv = torch.empty_like(v)
+    ws = None
     if ds_path:
         ws_bytes = int(L.sdpa_hip_bwd_workspace_bytes_full(dt, B, S_q, S_kv, D_qk, D_v,
                                                            int(bool(causal_mask))))
-    else:
+        ws = _workspace(torch, max(ws_bytes, 1), q.device)
+    if ws is None:
         ws_bytes = int(L.sdpa_hip_bwd_workspace_bytes(B, S_q))
-    ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=q.device)
+        ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=q.device)
     rc = L.sdpa_hip_bwd(dt, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                         stats.data_ptr(), d_o.data_ptr(), dq.data_ptr(), dk.data_ptr(),
                         dv.data_ptr(), ws.data_ptr(), ws_bytes, B, S_q, S_kv, D_qk, D_v,
