@@ -58,14 +58,14 @@ def test_small_forward(pkg, O, case):
 
 
 F32 = [
-    # B, S_q, S_kv, D_qk, D_v, causal, dropout, scale
-    (2, 129, 64, 64, 64, False, 0.1, 0.125),     # one block, a one-row tile
-    (1, 33, 2049, 128, 128, False, 0.0, 0.1),    # 32-key blocks, parts, a one-key tail
-    (2, 65, 65, 37, 5, True, 0.2, -0.2),         # element loads, negated scale
-    (2, 200, 200, 32, 128, True, 0.1, 0.0),      # scale 0
-    (3, 1, 700, 128, 64, False, 1.5, 0.1),       # every element dropped
-    (1, 17, 8193, 40, 36, False, 0.1, 0.16),     # the sequential fp32 sums (more than 8192 keys)
-    (1, 33, 8225, 126, 6, False, 0.0, 0.09),     # the same with rows of no whole chunks
+    # B, S_q, S_kv, D_qk, D_v, causal, dropout, scale; whether the keys are divided
+    (2, 129, 64, 64, 64, False, 0.1, 0.125, False),     # one block, a one-row tile
+    (1, 33, 2049, 128, 128, False, 0.0, 0.1, True),     # 32-key blocks, parts, a one-key tail
+    (2, 65, 65, 37, 5, True, 0.2, -0.2, False),         # element loads, negated scale
+    (2, 200, 200, 32, 128, True, 0.1, 0.0, True),       # scale 0
+    (3, 1, 700, 128, 64, False, 1.5, 0.1, True),        # every element dropped
+    (1, 17, 8193, 40, 36, False, 0.1, 0.16, False),     # the sequential fp32 sums (more than 8192 keys)
+    (1, 33, 8225, 126, 6, False, 0.0, 0.09, False),     # the same with rows of no whole chunks
 ]
 
 
@@ -73,12 +73,13 @@ F32 = [
 def test_f32_forward(pkg, O, case):
     """The fp32 forward on the bf16 matrix cores: o within 1e-5 and, where
     keys are divided, the undivided form as well."""
-    B, S_q, S_kv, D_qk, D_v, causal, p, scale = case
+    B, S_q, S_kv, D_qk, D_v, causal, p, scale, divided = case
     c = Cfg("f32_fwd", "f32", B, S_q, S_kv, D_qk, D_v, causal, p, scale, 3, 17)
     q, k, v, _ = make_inputs(c)
     o_ref, s_ref = O.sdpa_fwd_gate(q, k, v, **oracle_kw(c))
     L = pkg.library()
     want = L.sdpa_hip_fwd_workspace_bytes(0, B, S_q, S_kv, D_qk, D_v, int(causal))
+    assert (want > 0) == divided
     t = [_t(a) for a in (q, k, v)]
     for ws_bytes in {want, 0}:
         ws = torch.empty((max(want, 1),), dtype=torch.uint8, device=t[0].device)
