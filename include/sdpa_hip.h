@@ -111,7 +111,10 @@ int sdpa_hip_fwd(int dtype, const void* q, const void* k, const void* v, void* o
  * of a tile are divided over several workgroups, which needs
  * sdpa_hip_fwd_workspace_bytes(...) bytes of device memory, 16-byte aligned,
  * for their partial results; 0 where nothing is divided.  With less (or
- * none) the call runs undivided, as sdpa_hip_fwd does.                      */
+ * none) the call runs undivided, as sdpa_hip_fwd does.  The sums of a divided
+ * row are added in another order: its last bits differ between the two forms,
+ * and, as the division goes by the number of tiles, between batch sizes.  Each
+ * call repeats to the bit.                                                  */
 size_t sdpa_hip_fwd_workspace_bytes(int dtype, int B, int S_q, int S_kv, int D_qk, int D_v,
                                     int causal_mask);
 
@@ -165,11 +168,12 @@ int sdpa_hip_bwd_dkdv(int dtype, const void* q, const void* k, const void* v, co
 size_t sdpa_hip_bwd_workspace_bytes_ds(int dtype, int B, int S_q, int S_kv, int D_qk, int D_v,
                                        int causal_mask);
 
-/* The largest workspace sdpa_hip_bwd makes use of: that of the dS path, or
- * for float16 shapes without one whose query side has few tiles (a few
- * queries against a long memory) the per-row workspace plus the partial dQ
- * of the workgroups that then share a tile's keys; elsewhere the per-row
- * workspace.  Any smaller workspace works as described above.               */
+/* The largest workspace sdpa_hip_bwd makes use of: that of the dS path; or,
+ * for shapes without one that have few tiles, the per-row workspace plus the
+ * partial sums of the workgroups that then share a tile: dQ of a tile's keys
+ * (a few queries against a long memory) and, float32, dK and dV of a tile's
+ * queries; elsewhere the per-row workspace.  Any smaller workspace works as
+ * described above (with the note on divided sums at sdpa_hip_fwd_ws).       */
 size_t sdpa_hip_bwd_workspace_bytes_full(int dtype, int B, int S_q, int S_kv, int D_qk, int D_v,
                                          int causal_mask);
 

@@ -14,7 +14,7 @@
 //
 // D <= 64 may also be a multiple of 4 only (P4, keep4), which the large
 // kernels' copies do not take: the register-staged kernels served such shapes
-// (step of B 20, S 400, D 32/4, dropout: 87 -> 32 us).
+// (step of B 20, S 400, D 32/4, dropout: 87 -> 33 us).
 //
 // Element semantics are those of the large kernels (sdpa_bwd.hip restates the
 // reference's, sdpa/sdpa_bwd.cu.cc:130-170, 291-327).

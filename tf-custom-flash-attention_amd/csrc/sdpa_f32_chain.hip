@@ -1,5 +1,5 @@
 // sdpa_f32_chain.hip -- the fp32 forward and dK/dV on
-// v_mfma_f32_32x32x2_f32, for the shapes of fp32_chain() (sdpa_parts.h); all
+// v_mfma_f32_32x32x2_f32, for the shapes of fp32_chain_fwd() and fp32_chain() (sdpa_parts.h); all
 // others run on the bf16 matrix cores (sdpa_f32_fwd.hip, sdpa_f32_dkdv.hip).
 //
 // The gradient leaves out weights P <= 1e-6, a step, and a weight within a

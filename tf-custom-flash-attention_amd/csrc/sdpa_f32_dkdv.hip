@@ -11,13 +11,14 @@
 // in its first half S and P beside dP and the dS role's share of the staging,
 // then (P, with the dropout decision in its sign, has gone through LDS) dV and
 // the P role's share beside dS and dK.  The query blocks of a tile may be
-// divided over workgroups (bwd_f32_kv_parts), whose sums a second kernel adds.
+// divided over workgroups (bwd_parts), whose sums a second kernel adds.
 //
 // What bounds it: VALU work (cutting, elements) that overlaps the MFMAs in
-// part; the matrix cores are busy about half of the time.  B 64, S_q 512,
-// S_kv 16384, D 128/64, with the dS stores: 3.53 -> 2.50 ms against
-// v_mfma_f32_32x32x2_f32, error of dK against 64 bits 1.2e-6 -> 1.1e-6.  The
-// dS role one block behind (three stages, one barrier a block) measured 2.61.
+// part; the matrix cores are busy 46%.  B 64, S_q 512, D 128/64, with the dS
+// stores: 1.19 ms at 8192 keys, 1.87 ms on v_mfma_f32_32x32x2_f32 at 8224 (70%
+// busy; sdpa_f32_chain.hip, which takes over there), error of dK against 64
+// bits 8.2e-7 and 9.1e-7; D 64 without them 0.82 and 1.33 ms.  The dS role one
+// block behind (three stages, one barrier a block) was 4% slower.
 #include <type_traits>
 
 #include "sdpa_bf3.h"

@@ -10,12 +10,13 @@
 //   S^T = K Q^T, online softmax, O^T += V^T P~^T  (P~ cut in registers).
 // The keys of a tile may be divided over workgroups (fwd_f32_parts).
 //
-// What bounds it: VALU work (420 instructions per wave and 32 keys at
+// What bounds it: VALU work (410 instructions per wave and 32 keys at
 // 128/64: cutting, softmax) beside 72 MFMAs, which the two waves of a SIMD
-// overlap only in part (the matrix cores are busy 56%).  B 64, S_q 512, S_kv
-// 16384, D 128/64: 1.76 -> 1.08 ms against v_mfma_f32_32x32x2_f32 (which was
-// 75% busy), error against 64 bits 2.3e-6 -> 1.6e-6 (fewer roundings per
-// sum).  Not faster: staging one half of the waves earlier, operands read
+// overlap only in part (the matrix cores are busy 52%).  B 64, S_q 512, D
+// 128/64: 0.58 ms at 8192 keys, 0.89 ms on v_mfma_f32_32x32x2_f32 at 8224
+// (73% busy; sdpa_f32_chain.hip, which takes over there), error against 64
+// bits 1.1e-6 and 1.7e-6 (fewer roundings per sum); D 64: 0.41 and 0.65 ms.
+// Not faster: staging one half of the waves earlier, operands read
 // ahead, two workgroups of four waves per CU instead of one of eight.
 #include <type_traits>
 
@@ -103,7 +104,8 @@ void sdpa_fwd_f32_bf3_kernel(const FwdParams p, const int win) {
         kst.load(Kb, n0, S_kv - n0, D_qk, D_qk, tid);
         vst.load(Vb, n0, S_kv - n0, D_v, D_v, tid);
     };
-    // INF: again, for infinities in V (sdpa_bf3.h)
+    // INF: again, for infinities in V (sdpa_bf3.h).  Looking for them in V as it
+    // is staged, or in the loop, cost 3 to 10%; the sums show them for nothing.
     auto pass = [&](auto inf) {
         constexpr bool INF = decltype(inf)::value;
 #pragma unroll

@@ -76,7 +76,7 @@ hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, bool half4, int
 // every tensor 16-byte aligned.
 hipError_t launch_fwd_f16_dma(const FwdParams& p, hipStream_t stream);
 // The same for grids too small to fill the chip (sdpa_f16_fwd_small.hip);
-// p.div and the part buffers as planned by fwd_plan().
+// p.parts and the part buffers as planned by fwd_plan().
 hipError_t launch_fwd_f16_wave(const FwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_f16_dma(const BwdParams& p, int phases, hipStream_t stream);
 // dQ phase of launch_bwd_f16_dma (sdpa_f16_dq.hip)
@@ -108,7 +108,8 @@ hipError_t launch_bwd_dkdv_f32(const BwdParams& p, bool vec, hipStream_t stream)
 hipError_t launch_bwd_rows_f32(const BwdParams& p, hipStream_t stream);
 hipError_t launch_bwd_dq_ds_f32(const BwdParams& p, hipStream_t stream);
 
-// The fp32 forward and dK/dV of the shapes of fp32_chain() (sdpa_f32_chain.hip).
+// The fp32 forward of the shapes of fp32_chain_fwd() and dK/dV of those of
+// fp32_chain() (sdpa_f32_chain.hip).
 hipError_t launch_fwd_f32_chain(const FwdParams& p, bool vec, hipStream_t stream);
 hipError_t launch_bwd_dkdv_f32_chain(const BwdParams& p, bool vec, hipStream_t stream);
 
