@@ -500,7 +500,9 @@ struct BwdQF32Cfg {
     static constexpr int waves() { return (DQK == 128 && (DV == 128 || (DV == 64 && !VEC))) ? 1 : 2; }
 };
 
-template <int DQK, int DV, bool VEC, bool DROP>
+// DIV: a tile's keys divided over p.parts workgroups (an instantiation of its
+// own: the range in registers cost the undivided kernel 3 to 6%).
+template <int DQK, int DV, bool VEC, bool DROP, bool DIV>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(BwdQF32Cfg<DQK, DV>::template waves<VEC, DROP>(),
                                    BwdQF32Cfg<DQK, DV>::template waves<VEC, DROP>())))
@@ -515,10 +517,10 @@ void sdpa_bwd_dq_f32_kernel(const BwdParams p) {
     const int l32 = lane & 31, hh = lane >> 5;
     const int B = p.s.B, S_q = p.s.S_q, S_kv = p.s.S_kv, D_qk = p.s.D_qk, D_v = p.s.D_v;
     const bool causal = p.c.causal != 0;
-    const int np = p.parts, items = (S_q + BM - 1) / BM * np;
+    const int np = DIV ? p.parts : 1, items = (S_q + BM - 1) / BM * np;
     int b, it;
     map_tile(blockIdx.x, B, items, causal, b, it);
-    const int qt = it / np, part = it - qt * np;
+    const int qt = DIV ? it / np : it, part = DIV ? it - qt * np : 0;
     const int q0 = qt * BM, qw0 = q0 + wave * 32, my_q = qw0 + l32;
     const size_t row_q = (size_t)b * S_q + my_q;
 
@@ -558,7 +560,7 @@ void sdpa_bwd_dq_f32_kernel(const BwdParams p) {
 
     const int kv_end = causal ? min(S_kv, q0 + BM) : S_kv;
     const int blocks = (kv_end + BN - 1) / BN;  // of them this part's: [lo, nblk)
-    const int lo = part_begin(blocks, part, np), nblk = part_begin(blocks, part + 1, np);
+    const int lo = DIV ? part_begin(blocks, part, np) : 0, nblk = DIV ? part_begin(blocks, part + 1, np) : blocks;
     const bool wave_live = qw0 < S_q;
     const int wave_last_q = min(qw0 + 31, S_q - 1);
     const uint64_t st_base = DROP ? lcg_state(p.c.seed_offset, row_q, (uint64_t)S_kv, 4 * hh) : 0;
@@ -643,8 +645,8 @@ void sdpa_bwd_dq_f32_kernel(const BwdParams p) {
     }
 
     if (row_ok) {
-        const float sc = np > 1 ? 1.f : p.c.scale;
-        float* dQb = np > 1 ? p.part_dq + ((size_t)part * B * S_q + row_q) * D_qk : static_cast<float*>(p.dq) + row_q * D_qk;
+        const float sc = DIV ? 1.f : p.c.scale;
+        float* dQb = DIV ? p.part_dq + ((size_t)part * B * S_q + row_q) * D_qk : static_cast<float*>(p.dq) + row_q * D_qk;
 #pragma unroll
         for (int dt = 0; dt < DQK / 32; ++dt)
 #pragma unroll
@@ -697,7 +699,14 @@ hipError_t launch_bwd(const BwdParams& p, DType dtype, bool vec, bool half4, int
                             if (DQK == 128 || DV == 128 || fp32_chain(p.s)) {
                                 using CQ = BwdQF32Cfg<DQK, DV>;
                                 const unsigned gq = (unsigned)(((S_q + CQ::BM - 1) / CQ::BM) * p.parts * B);
-                                err = launch_kernel<sdpa_bwd_dq_f32_kernel<DQK, DV, V, D>>(gq, CQ::NT, CQ::LDS_BYTES, stream, p);
+                                if (p.parts == 1) {
+                                    err = launch_kernel<sdpa_bwd_dq_f32_kernel<DQK, DV, V, D, false>>(gq, CQ::NT, CQ::LDS_BYTES, stream, p);
+                                } else {
+                                    if constexpr (DQK <= 64 && DV <= 64)
+                                        err = launch_kernel<sdpa_bwd_dq_f32_kernel<DQK, DV, V, D, true>>(gq, CQ::NT, CQ::LDS_BYTES, stream, p);
+                                    else
+                                        err = hipErrorInvalidValue;
+                                }
                             } else {
                                 err = launch_bwd_dq_f32(p, V, stream);
                             }
