@@ -346,6 +346,7 @@ BWD = [
     ("f32", 2, 5, 8200, 64, 64, False, 0.1, 2),     # the same for few queries, dQ in parts
     ("f32", 1, 16, 9001, 37, 5, False, 0.0, 2),     # and with element loads
     ("f32", 1, 33, 8225, 128, 64, False, 0.0, 1),   # the same, dS path
+    ("f32", 1, 70, 8193, 5, 64, False, 0.2, 1),     # its dK/dV at D <= 64: element loads, a one-key tile
 ]
 
 

@@ -208,6 +208,208 @@ void sdpa_fwd_f32_chain_kernel(const FwdParams p) {
 }
 
 // ---------------------------------------------------------------------------
+// dK/dV at D <= 64: four waves, each all of its 32 keys (K, V, dK and dV fit
+// in one wave's registers there).  Against the split roles below: B 16, S_q
+// 512, S_kv 9000, D 32 256 -> 227 us, D 64 423 -> 398.
+// ---------------------------------------------------------------------------
+template <int DQK, int DV>
+struct DkvWaveChainCfg {
+    static constexpr int NT = 256, BKV = 128, BQ = 32;
+    static constexpr int QS = DQK + 4, OS = DV + 4;
+    static constexpr int QT = BQ * QS, OT = BQ * OS;
+    static constexpr int STAGE = QT + OT + 2 * BQ;  // floats: Q, dO, stats2, delta
+    static constexpr size_t LDS_BYTES = 2 * (size_t)STAGE * sizeof(float);
+};
+
+template <int DQK, int DV, bool VEC, bool DROP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void sdpa_bwd_dkdv_f32_chain_wave_kernel(const BwdParams p) {
+    using Cfg = DkvWaveChainCfg<DQK, DV>;
+    constexpr int BKV = Cfg::BKV, BQ = Cfg::BQ, QS = Cfg::QS, OS = Cfg::OS;
+    constexpr int HQ = DQK / 2, HV = DV / 2;
+    float* lds = reinterpret_cast<float*>(smem);
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l32 = lane & 31, hh = lane >> 5;
+    const int B = p.s.B, S_q = p.s.S_q, S_kv = p.s.S_kv, D_qk = p.s.D_qk, D_v = p.s.D_v;
+    const bool causal = p.c.causal != 0;
+    const int tiles = (S_kv + BKV - 1) / BKV;
+    int b, kt;
+    map_q_tile(blockIdx.x, B, tiles, false, b, kt);
+    const int k0 = kt * BKV, kw0 = k0 + wave * 32, my_k = kw0 + l32;
+    const bool key_ok = my_k < S_kv;
+
+    const float* Qb = static_cast<const float*>(p.q) + (size_t)b * S_q * D_qk;
+    const float* dOb = static_cast<const float*>(p.d_o) + (size_t)b * S_q * D_v;
+    const float* Kb = static_cast<const float*>(p.k) + (size_t)b * S_kv * D_qk;
+    const float* Vb = static_cast<const float*>(p.v) + (size_t)b * S_kv * D_v;
+    const float* statsb = p.stats + (size_t)b * S_q;
+    const float* deltab = p.delta + (size_t)b * S_q;
+
+    float kf[HQ], vf[HV];
+#pragma unroll
+    for (int u = 0; u < HQ / 4; ++u) {
+        const floatx4 f = __builtin_bit_cast(floatx4, load_row_chunk<float, VEC>(Kb, my_k, S_kv, HQ * hh + 4 * u, D_qk, D_qk));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kf[4 * u + e] = f[e];
+    }
+#pragma unroll
+    for (int u = 0; u < HV / 4; ++u) {
+        const floatx4 f = __builtin_bit_cast(floatx4, load_row_chunk<float, VEC>(Vb, my_k, S_kv, HV * hh + 4 * u, D_v, D_v));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vf[4 * u + e] = f[e];
+    }
+    prologue_loads_landed();
+
+    const int q_begin = causal ? (min(k0, S_q) / BQ) * BQ : 0;
+    const int nblk = (S_q - q_begin + BQ - 1) / BQ;
+    const bool wave_live = kw0 < S_kv;
+    const float sl2 = p.c.scale_log2;
+    const float ksc = p.c.keep_scale;
+    const uint64_t st_base = DROP ? lcg_state(p.c.seed_offset, (uint64_t)b * S_q + 4 * hh, (uint64_t)S_kv, my_k) : 0;
+    const uint64_t row_step = (uint64_t)S_kv * kLcgMul;
+    const uint32_t thr = p.c.drop_threshold;
+
+    floatx16 dkacc[DQK / 32], dvacc[DV / 32];
+#pragma unroll
+    for (int dt = 0; dt < DQK / 32; ++dt) dkacc[dt] = floatx16{};
+#pragma unroll
+    for (int dt = 0; dt < DV / 32; ++dt) dvacc[dt] = floatx16{};
+
+    TileStage<float, BQ, DQK, Cfg::NT, VEC> qst;
+    TileStage<float, BQ, DV, Cfg::NT, VEC> ost;
+    float fpre = 0.f;
+    auto load_rows = [&](int q0) {
+        qst.template load<false>(Qb, q0, S_q - q0, D_qk, D_qk, tid);
+        ost.template load<false>(dOb, q0, S_q - q0, D_v, D_v, tid);
+        if (tid < 2 * BQ) {
+            const int r = q0 + (tid & (BQ - 1));
+            if (tid < BQ) fpre = r < S_q ? statsb[r] * kLog2e : INFINITY;
+            else fpre = r < S_q ? deltab[r] : 0.f;
+        }
+    };
+    auto store_rows = [&](int s) {
+        float* base = lds + s * Cfg::STAGE;
+        qst.template store<QS>(base, tid);
+        ost.template store<OS>(base + Cfg::QT, tid);
+        if (tid < 2 * BQ) base[Cfg::QT + Cfg::OT + tid] = fpre;
+    };
+
+    if (nblk > 0) {
+        load_rows(q_begin);
+        store_rows(0);
+    }
+    __syncthreads();
+
+    for (int blk = 0; blk < nblk; ++blk) {
+        const int q0 = q_begin + blk * BQ;
+        const int cur = blk & 1;
+        const float* Qs = lds + cur * Cfg::STAGE;
+        const float* dOs = Qs + Cfg::QT;
+        const float* Fs = dOs + Cfg::OT;
+        const bool has_next = blk + 1 < nblk;
+        if (has_next) load_rows(q0 + BQ);
+
+        if (wave_live && (!causal || q0 + BQ - 1 >= kw0)) {
+            floatx16 sacc = floatx16{}, dpacc = floatx16{};
+#pragma unroll
+            for (int u = 0; u < HQ / 4; ++u) {
+                const floatx4 qq = *reinterpret_cast<const floatx4*>(Qs + l32 * QS + HQ * hh + 4 * u);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sacc = mfma_f32(qq[e], kf[4 * u + e], sacc);
+            }
+#pragma unroll
+            for (int u = 0; u < HV / 4; ++u) {
+                const floatx4 oo = *reinterpret_cast<const floatx4*>(dOs + l32 * OS + HV * hh + 4 * u);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dpacc = mfma_f32(oo[e], vf[4 * u + e], dpacc);
+            }
+            const bool need_mask = !key_ok || (causal && q0 < kw0 + 31);
+            const uint64_t st_blk = DROP ? st_base + (uint64_t)q0 * row_step : 0;
+            float pk[16], ds[16];
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const int rb = 8 * g4 + 4 * hh;
+                const floatx4 st4 = *reinterpret_cast<const floatx4*>(Fs + rb);
+                const floatx4 de4 = *reinterpret_cast<const floatx4*>(Fs + BQ + rb);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = 4 * g4 + e;
+                    float x = __builtin_fmaf(sacc[r], sl2, -st4[e]);
+                    if (need_mask) {
+                        const int q = q0 + rb + e;
+                        if (!key_ok || (causal && my_k > q)) x = -INFINITY;
+                    }
+                    const float pr = fast_exp2(x);
+                    const float p0 = pr > kEps ? pr : 0.f;
+                    float dpk = DROP ? dpacc[r] * ksc : dpacc[r];
+                    float pkk = p0;
+                    if constexpr (DROP) {
+                        const uint64_t off = (uint64_t)(8 * g4 + e) * row_step;
+                        const bool keep = lcg_keep(st_blk + off, thr);
+                        dpk = keep ? dpk : 0.f;
+                        pkk = keep ? p0 : 0.f;
+                    }
+                    pk[r] = pkk;
+                    ds[r] = p0 * (dpk - de4[e]);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int qrow = 8 * (r >> 2) + 4 * hh + (r & 3);
+#pragma unroll
+                for (int dt = 0; dt < DV / 32; ++dt)
+                    dvacc[dt] = mfma_f32(dOs[qrow * OS + 32 * dt + l32], pk[r], dvacc[dt]);
+#pragma unroll
+                for (int dt = 0; dt < DQK / 32; ++dt)
+                    dkacc[dt] = mfma_f32(Qs[qrow * QS + 32 * dt + l32], ds[r], dkacc[dt]);
+            }
+        }
+
+        if (has_next) store_rows(cur ^ 1);
+        __syncthreads();
+    }
+
+    if (key_ok) {
+        const float sc = p.c.scale;
+        float* dKb = static_cast<float*>(p.dk) + ((size_t)b * S_kv + my_k) * D_qk;
+        float* dVb = static_cast<float*>(p.dv) + ((size_t)b * S_kv + my_k) * D_v;
+#pragma unroll
+        for (int dt = 0; dt < DQK / 32; ++dt)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const int d0 = 32 * dt + 8 * g4 + 4 * hh;
+                floatx4 fv;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) fv[e] = dkacc[dt][4 * g4 + e] * sc;
+                if constexpr (VEC) {
+                    if (d0 < D_qk) *reinterpret_cast<floatx4*>(dKb + d0) = fv;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (d0 + e < D_qk) dKb[d0 + e] = fv[e];
+                }
+            }
+#pragma unroll
+        for (int dt = 0; dt < DV / 32; ++dt)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const int d0 = 32 * dt + 8 * g4 + 4 * hh;
+                floatx4 fv;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) fv[e] = dvacc[dt][4 * g4 + e] * ksc;
+                if constexpr (VEC) {
+                    if (d0 < D_v) *reinterpret_cast<floatx4*>(dVb + d0) = fv;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (d0 + e < D_v) dVb[d0 + e] = fv[e];
+                }
+            }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // dK/dV: two waves per group of 32 keys (P role: S, P~, dV; dS role: dP, dS,
 // dK, one query block behind), blocks of 32 queries in a ring of three stages.
 // ---------------------------------------------------------------------------
@@ -506,8 +708,15 @@ hipError_t launch_bwd_dkdv_f32_chain(const BwdParams& p, bool vec, hipStream_t s
                                                                                                  stream, p);
                     }
                     if (p.ds) return hipErrorInvalidValue;
-                    return launch_kernel<sdpa_bwd_dkdv_f32_chain_kernel<DQK, DV, V, D, false>>(n, Cfg::NT, Cfg::LDS_BYTES,
-                                                                                          stream, p);
+                    if constexpr (DQK == 128 || DV == 128) {
+                        return launch_kernel<sdpa_bwd_dkdv_f32_chain_kernel<DQK, DV, V, D, false>>(n, Cfg::NT, Cfg::LDS_BYTES,
+                                                                                              stream, p);
+                    } else {
+                        using CW = DkvWaveChainCfg<DQK, DV>;
+                        static_assert(CW::BKV == Cfg::BKV, "same grid");
+                        return launch_kernel<sdpa_bwd_dkdv_f32_chain_wave_kernel<DQK, DV, V, D>>(n, CW::NT, CW::LDS_BYTES,
+                                                                                            stream, p);
+                    }
                 });
             });
         });

@@ -262,7 +262,7 @@ void sdpa_fwd_f32_bf3_kernel(const FwdParams p, const int win) {
 hipError_t launch_fwd_f32(const FwdParams& p, bool vec, hipStream_t stream) {
     const int B = p.s.B, S_q = p.s.S_q;
     if (B == 0 || S_q == 0) return hipSuccess;
-    if (fp32_chain_fwd(p.s)) return launch_fwd_f32_chain(p, vec, stream);
+    if (fp32_chain_fwd(p.s, p.c.causal != 0)) return launch_fwd_f32_chain(p, vec, stream);
     return with_dim(p.s.D_qk, [&](auto dqk) {
         return with_dim(p.s.D_v, [&](auto dv) {
             return with_bool(vec, [&](auto v) {

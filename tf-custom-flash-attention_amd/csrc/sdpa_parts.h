@@ -69,7 +69,18 @@ inline int pad_dim(int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }
 // 16384, D 64 and 128, and S_q 4, S_kv 32768 (with the gradient there as well
 // 3, 7 and 20; the largest change of an element 7e-4 of the root mean square).
 inline bool fp32_chain(const AttnShape& s) { return s.S_kv > 8192; }
-inline bool fp32_chain_fwd(const AttnShape& s) { return fp32_chain(s) && s.S_q > 16; }
+// The forward also where few keys meet more than 256 tiles of 128 queries: two
+// of its workgroups of four waves share a CU and start sooner than one of
+// eight, and its blocks are of 32 keys.  Chain -> bf16 parts, us: B 100, S_q
+// 1000, D 64, 8 keys 23.4 -> 37.0, 64 keys 31.8 -> 39.0, 129 keys 56.7 -> 58.3,
+// 192 keys 65.6 -> 61.1; D 32, 129 keys 33.4 -> 39.0, 192 keys 37.2 -> 39.4, 256
+// keys 47.1 -> 45.9; B 600, causal, D 128, S 129 97 -> 117, S 192 126 -> 132.
+inline bool fp32_chain_fwd(const AttnShape& s, bool causal) {
+    const int few = causal || (s.D_qk <= 32 && s.D_v <= 32) ? 192 : 160;
+    const long long tiles = (long long)s.B * ((s.S_q + 127) / 128);
+    if (s.S_kv <= few && tiles > 256 && tiles < 1 << 24) return true;  // (its grid has one dimension)
+    return fp32_chain(s) && s.S_q > 16;
+}
 
 // Parts of the keys of a 128-query tile in the fp32 forward (sdpa_f32_fwd.hip).
 // A block (64 keys, 32 where both sides are 128 wide) takes about 0.0215 us
@@ -78,7 +89,7 @@ inline bool fp32_chain_fwd(const AttnShape& s) { return fp32_chain(s) && s.S_q >
 // S_kv 8000, D 64: 288 -> 22.6 (32 parts); B 64, S_q 64, S_kv 2000, D 128:
 // 194 -> 65 (4); B 24, S 700, D 64: 38 (1; in two parts 57: a second round).
 inline int fwd_f32_parts(int B, int S_q, int S_kv, int D_qk, int D_v, bool causal) {
-    if (fp32_chain_fwd(AttnShape{B, S_q, S_kv, D_qk, D_v})) return 1;
+    if (fp32_chain_fwd(AttnShape{B, S_q, S_kv, D_qk, D_v}, causal)) return 1;
     const int pq = pad_dim(D_qk), pv = pad_dim(D_v);
     const bool wide = pq == 128 && pv == 128;
     return least_time_parts((long long)B * ((S_q + 127) / 128), ((long long)S_kv + (wide ? 31 : 63)) / (wide ? 32 : 64),
