@@ -66,6 +66,9 @@ F32 = [
     (3, 1, 700, 128, 64, False, 1.5, 0.1, True),        # every element dropped
     (1, 17, 8193, 40, 36, False, 0.1, 0.16, False),     # the sequential fp32 sums (more than 8192 keys)
     (1, 33, 8225, 126, 6, False, 0.0, 0.09, False),     # the same with rows of no whole chunks
+    (257, 3, 31, 64, 64, False, 0.1, -0.125, False),    # few keys against more than 256 tiles: the fp32 instruction
+    (129, 160, 160, 37, 128, True, 0.2, 0.1, False),    # the same, causal, within its lengths
+    (260, 2, 161, 64, 33, False, 0.0, 0.125, False),    # one key more than it takes without the mask
 ]
 
 
@@ -123,6 +126,15 @@ def test_f32_grid_of_more_threads_than_one_dimension(pkg):
     assert (s - (q * k).sum(2) * 0.5).abs().max().item() <= 1e-4
     assert (dv - d_o).abs().max().item() <= 1e-4
     assert dq.abs().max().item() <= 1e-4 and dk.abs().max().item() <= 1e-4
+    # the forward of 512 threads takes more than 160 keys there
+    del o, s, dq, dk, dv, v, d_o
+    q = q[..., :1].contiguous()
+    k, v = (torch.randn((B, 161, 1), generator=g, device="cuda") for _ in range(2))
+    o, _ = pkg.sdpa(q, k, v, scale=0.5)
+    for i in range(0, B, 1 << 20):
+        j = slice(i, i + (1 << 20))
+        ref = (torch.softmax(q[j] * k[j] * 0.5, 1) * v[j]).sum(1, keepdim=True)
+        assert (o[j] - ref).abs().max().item() <= 1e-5
 
 
 @pytest.mark.parametrize("dtype,D", [(torch.float16, 64), (torch.float32, 64), (torch.float16, 128)])

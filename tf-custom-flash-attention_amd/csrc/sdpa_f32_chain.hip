@@ -19,6 +19,9 @@
 // features [h D/2, (h+1) D/2), so operands are read as float4 runs;
 // reductions over keys or queries pair k-step r of lane-half h with row 8
 // (r/4) + 4h + r%4 of the 32-row accumulator tile.
+//
+// The forward serves few keys against many tiles as well, where it is the faster
+// one (fp32_chain_fwd()).
 #include <type_traits>
 
 #include "sdpa_dma.h"
